@@ -291,6 +291,13 @@ namespace ormi::hip {
             bool off32 = false;
             int vec = 1;
             int vec_dim = -1;  // dim whose coordinate advances by VEC
+            // The vector dim's extent is not a multiple of VEC: its last group
+            // starts at extent - VEC and so repeats up to VEC - 1 elements of
+            // the group before (argument E is that start). No access passes
+            // the row's end, and a map stores the repeated elements' bits twice.
+            bool tail = false;
+            // Leaves read VEC-wide from addresses that are only element-aligned.
+            std::vector<bool> unaligned;
             int rows = 0;      // map tile alignment to the last dim (plan_map_multi)
             // Non-temporal hint on the loads of streamed leaves: those with no
             // zero stride in the canonical (size-1-free) dims, whose elements
@@ -318,6 +325,7 @@ namespace ormi::hip {
             // Output dtypes of a map: bf16 and fp16 share a storage type, so the
             // argument list alone does not tell their stores apart.
             std::vector<DType> out_dtypes;
+            std::vector<bool> out_unaligned;  // outputs whose groups are only element-aligned (map)
             ArgList args;
             std::unique_ptr<std::ostringstream> body_;  // created when a source is generated
 
@@ -345,20 +353,66 @@ namespace ormi::hip {
             bool leaf_vec_ok(size_t L, int d) const {
                 if (scalar[L]) return true;
                 const long long s = c.st[L][d];
-                if (s == 0) return true;
-                if (s != 1 || !vector_dtype(e.leaves[L].dtype)) return false;
+                return s == 0 || (s == 1 && vector_dtype(e.leaves[L].dtype));
+            }
+            // ... and every such group starts on a multiple of its own size.
+            bool leaf_aligned(size_t L, int d) const {
+                if (scalar[L] || c.st[L][d] == 0) return true;
+                if (tail) return false;
                 for (size_t k = 0; k < c.dims.size(); ++k)
                     if ((int)k != d && c.st[L][k] % 4 != 0) return false;
                 return ((uintptr_t)e.leaves[L].ptr % (4 * dtype_size(e.leaves[L].dtype))) == 0;
             }
 
-            void choose_vec(int d) {
+            // Four elements per group wherever every operand is unit-stride (or
+            // constant) along dim d, also from addresses and row lengths that
+            // are not multiples of the group: gfx950 reads 16 (or 8) bytes per
+            // lane from any element address, and a wave's lanes still cover one
+            // contiguous run, at one cache line more. Measured on C2's chain in
+            // bfloat16: 6001 x 2047 26.7 us with one element per lane, 15.4 in
+            // groups, the time of 6001 x 2048 (both bound by the arithmetic). ragged_ok: the
+            // caller handles an extent that is not a multiple of four (tail).
+            static constexpr long long kRaggedMin = 256 * 4 * 64;
+            void choose_vec(int d, bool ragged_ok) {
                 vec = 1;
                 vec_dim = d;
-                if (d < 0 || c.dims[d].size % 4 != 0) return;
+                tail = false;
+                unaligned.assign(e.leaves.size(), false);
+                if (d < 0) return;
+                const long long n = c.dims[d].size;
+                if (n < 4 || (n % 4 != 0 && !ragged_ok)) return;
                 for (size_t L = 0; L < e.leaves.size(); ++L)
                     if (!leaf_vec_ok(L, d)) return;
+                tail = n % 4 != 0;
+                bool any = tail;
+                for (size_t L = 0; L < e.leaves.size(); ++L) {
+                    unaligned[L] = !leaf_aligned(L, d);
+                    any = any || unaligned[L];
+                }
+                // Small ragged kernels keep one element per lane: with fewer
+                // elements than the chip's SIMDs have lanes, groups of four only
+                // serialize the arithmetic (a 4095-element power: 3.7 us, in
+                // groups 5.4).
+                long long numel = 1;
+                for (auto& x : c.dims) numel *= x.size;
+                if (any && numel < kRaggedMin) {
+                    tail = false;
+                    unaligned.assign(e.leaves.size(), false);
+                    return;
+                }
                 vec = 4;
+            }
+            // Groups of a dim (elements, where it is not the vector dim).
+            long long groups(int d) const { return d == vec_dim ? (c.dims[d].size + vec - 1) / vec : c.dims[d].size; }
+            // First element of the vector dim's group `q`.
+            std::string group_start(const std::string& q) const {
+                if (!tail) return vec > 1 ? "(" + q + ") * " + std::to_string(vec) : q;
+                const std::string x = "(" + q + ") * " + std::to_string(vec);
+                return "(" + x + " < (" + idx() + ")E ? " + x + " : (" + idx() + ")E)";
+            }
+            // Vector type of a group of `dt` values.
+            std::string group_type(DType dt, bool any_address) const {
+                return std::string(dt == DType::Float32 ? "ormi_f4" : "ormi_u16x4") + (any_address ? "u" : "");
             }
 
             // 32-bit index arithmetic when every index the kernel forms (element
@@ -393,13 +447,14 @@ namespace ormi::hip {
             // Size (in VEC groups for the vector dim) and fastdiv magic of each dim.
             void declare_dims() {
                 for (size_t d = 0; d < c.dims.size(); ++d) {
-                    const long long n = (int)d == vec_dim ? c.dims[d].size / vec : c.dims[d].size;
+                    const long long n = groups((int)d);
                     args.i64("D", n, (int)d);
                     if (idx32) {
                         const FastDiv f = make_fastdiv((uint32_t)n);
                         args.i64("M", (long long)((uint64_t)f.m | ((uint64_t)f.s << 32)), (int)d);
                     }
                 }
+                if (tail) args.i64("E", c.dims[vec_dim].size - vec);
             }
 
             // Runtime strides for the dims where they are neither 0 nor 1.
@@ -438,7 +493,10 @@ namespace ormi::hip {
                 }
                 o << ind << "  c" << dims[0] << " = rem_; }\n";
                 for (int d : dims)
-                    if (d == vec_dim && vec > 1) o << ind << "c" << d << " *= " << vec << ";\n";
+                    if (d == vec_dim && vec > 1) {
+                        const std::string cd = "c" + std::to_string(d);
+                        o << ind << cd << " = " << group_start(cd) << ";\n";
+                    }
             }
 
             void declare_coords(std::ostringstream& o, const std::string& ind, const std::vector<int>& dims) {
@@ -464,9 +522,9 @@ namespace ormi::hip {
                 const bool unit = vec > 1 && c.st[L][vec_dim] == 1;
                 const bool nt = nt_loads && streamed(L);
                 if (unit) {
-                    const char* vt = dt == DType::Float32 ? "ormi_f4" : "ormi_u16x4";
-                    const std::string addr = elem_ptr(std::string("const ") + vt + "*", p, off, dtype_size(dt), true);
-                    o << ind << "{ const " << vt << " v_ = " << (nt ? "__builtin_nontemporal_load(" + addr + ")" : "*" + addr) << ";";
+                    const std::string vt = group_type(dt, unaligned[L]);
+                    const std::string addr = elem_ptr("const " + vt + "*", p, off, dtype_size(dt), true);
+                    o << ind << "{ const " << group_type(dt, false) << " v_ = " << (nt ? "__builtin_nontemporal_load(" + addr + ")" : "*" + addr) << ";";
                     for (int k = 0; k < vec; ++k) {
                         const std::string ek = "v_[" + std::to_string(k) + "]";
                         o << " " << dst << "[" << k << "] = " << (dt == DType::Float32 ? ek : to_f32(dt, ek)) << ";";
@@ -686,6 +744,9 @@ namespace ormi::hip {
             append_int(s, g.vec);
             s += ',';
             append_int(s, g.vec_dim);
+            if (g.tail) s += 't';
+            for (bool u : g.unaligned) s += u ? 'u' : 'a';
+            for (bool u : g.out_unaligned) s += u ? 'u' : 'a';
             s += g.off32 ? ",32u," : g.idx32 ? ",32," : ",64,";
             append_int(s, g.rows);
             s += '|';
@@ -824,13 +885,17 @@ namespace ormi::hip {
             for (auto& s : g.c.st) s.push_back(0);
         }
         const int n = (int)g.c.dims.size();
-        g.choose_vec(n - 1);
-        for (size_t r = 0; r < nout; ++r)
-            if (!vector_dtype(out_dtypes[r]) || ((uintptr_t)outs[r] % 16) != 0) g.vec = 1;
+        bool vec_outs = true;
+        for (size_t r = 0; r < nout; ++r) vec_outs = vec_outs && vector_dtype(out_dtypes[r]);
+        g.choose_vec(vec_outs ? n - 1 : -1, true);
+        g.vec_dim = n - 1;
+        g.out_unaligned.assign(nout, false);
+        for (size_t r = 0; r < nout; ++r) g.out_unaligned[r] = g.vec > 1 && (g.tail || ((uintptr_t)outs[r] % 16) != 0);
         long long numel = 1;
         for (auto& d : g.c.dims) numel *= d.size;
         g.choose_nt_loads(tn.map_nt_loads, numel);
-        const long long G = numel / g.vec;
+        const long long last = g.c.dims[n - 1].size;
+        const long long G = last > 0 ? numel / last * g.groups(n - 1) : 0;
         const long long tile = (long long)block * unroll;
         const long long tiles = (G + tile - 1) / tile;
         long long grid = std::max(1LL, std::min(tiles, (long long)std::max(cu, 1) * tn.map_blocks_per_cu));
@@ -857,7 +922,7 @@ namespace ormi::hip {
         //          operands once for all its rows. The grid is a multiple of NW,
         //          so a block keeps its window and loads them once per block.
         const int n_last = n - 1;
-        const long long Dl = g.c.dims[n_last].size / g.vec;
+        const long long Dl = g.groups(n_last);
         if (tn.map_rows && g.idx32 && n >= 2 && Dl > 0) {
             if (tile == Dl) g.rows = 3;
             else if (tile % Dl == 0) g.rows = 1;
@@ -961,9 +1026,9 @@ namespace ormi::hip {
                 if (rows == 1) {
                     b << "    const " << t << " q = (" << t << ")ormi_fdiv((unsigned)l_, (unsigned)" << Mn << ", (unsigned)(" << Mn
                       << " >> 32));\n";
-                    b << "    q_[u] = q;\n    cl_[u] = (l_ - q * (" << t << ")" << Dn << ") * " << V << ";\n";
+                    b << "    q_[u] = q;\n    cl_[u] = " << g.group_start("l_ - q * (" + t + ")" + Dn) << ";\n";
                 } else {
-                    b << "    cl_[u] = l_ * " << V << ";\n";
+                    b << "    cl_[u] = " << g.group_start("l_") << ";\n";
                 }
                 b << "  }\n";
                 g.declare_leaf_regs(b, "  ", unroll, hoist);
@@ -1000,7 +1065,7 @@ namespace ormi::hip {
                 g.decompose(b, "    ", "row", outer);
                 g.declare_leaf_regs(b, "    ", unroll);
                 b << "#pragma unroll\n    for (int u = 0; u < " << unroll << "; ++u) {\n";
-                b << "      const " << t << " " << cl << " = (col0 + " << lane << ") * " << V << ";\n";
+                b << "      const " << t << " " << cl << " = " << g.group_start("col0 + " + lane) << ";\n";
                 load_all("      ", in_loop);
                 b << "    }\n";
             } else if (rows == 4) {
@@ -1008,7 +1073,7 @@ namespace ormi::hip {
                 // mod NW) is the same in every tile it visits; its rows advance
                 // by gridDim.x / NW tiles of `unroll` rows.
                 b << "  const " << t << " col0 = ((" << t << ")blockIdx.x % (" << t << ")NW) * " << block << ";\n";
-                b << "  const " << t << " " << cl << " = (col0 + " << tid << ") * " << V << ";\n";
+                b << "  const " << t << " " << cl << " = " << g.group_start("col0 + " + tid) << ";\n";
                 g.declare_leaf_regs(b, "  ", unroll, hoist);
                 b << "  {\n    const int u = 0;\n";
                 load_all("    ", hoist);
@@ -1052,14 +1117,29 @@ namespace ormi::hip {
             if (guard) b << "      if (go < (" << t << ")G) {\n";
             const std::string ind = guard ? "        " : "      ";
             const bool nt = tn.map_nt_stores;
+            // First element of the group in the (contiguous) outputs.
+            std::string at = "go * " + std::to_string(V);
+            if (g.tail) {
+                b << ind;
+                if (n == 1) {
+                    b << "const " << t << " eo = " << g.group_start("go") << ";\n";
+                } else {
+                    b << "const " << t << " ro_ = ";
+                    if (g.idx32) b << "(" << t << ")ormi_fdiv((unsigned)go, (unsigned)" << Mn << ", (unsigned)(" << Mn << " >> 32))";
+                    else b << "go / " << Dn;
+                    b << ";\n" << ind << "const " << t << " eo = ro_ * ((" << t << ")E + " << V << ") + "
+                      << g.group_start("go - ro_ * (" + t + ")" + Dn) << ";\n";
+                }
+                at = "eo";
+            }
             for (size_t r = 0; r < nout; ++r) {
                 const DType odt = out_dtypes[r];
                 if (V == 4) {
-                    const char* vt = odt == DType::Float32 ? "ormi_f4" : "ormi_u16x4";
-                    std::string val = std::string(vt) + "{";
+                    const std::string vt = g.group_type(odt, g.out_unaligned[r]);
+                    std::string val = g.group_type(odt, false) + "{";
                     for (int q = 0; q < 4; ++q) val += (q ? ", " : "") + from_f32(odt, res(r) + "[" + std::to_string(q) + "]");
                     val += "}";
-                    const std::string addr = g.elem_ptr(std::string(vt) + "*", out_name(r), "go * 4", dtype_size(odt), false);
+                    const std::string addr = g.elem_ptr(vt + "*", out_name(r), at, dtype_size(odt), false);
                     if (nt) b << ind << "__builtin_nontemporal_store(" << val << ", " << addr << ");\n";
                     else b << ind << "*" << addr << " = " << val << ";\n";
                 } else {
@@ -1105,7 +1185,11 @@ namespace ormi::hip {
         if (R >= (1ll << 31)) throw std::runtime_error("HIP reduce: reduced extent above 2^31 elements.");
         const std::vector<int> od = dims_of(g.c, G_O), rd = dims_of(g.c, G_R), id = dims_of(g.c, G_I);
         const bool column = !id.empty();
-        g.choose_vec(column ? id.back() : (rd.empty() ? -1 : rd.back()));
+        // A ragged vector dim must be the only dim of its group: positions
+        // within the group are then group starts plus the lane's slot.
+        // Fewer than 16 ragged columns keep one lane per column.
+        if (column) g.choose_vec(id.back(), id.size() == 1 && I >= 16);
+        else g.choose_vec(rd.empty() ? -1 : rd.back(), rd.size() == 1);
 
         ReducePlan plan;
         KernelLaunch& k = plan.first;
@@ -1117,7 +1201,7 @@ namespace ormi::hip {
         if (!column) {
             // ---------------------------------------------------------- row --
             const int RU = tn.row_unroll;
-            const long long RG = R / V;
+            const long long RG = (R + V - 1) / V;
             long long P = 1;
             const long long target_waves = (long long)std::max(cu, 1) * 32;
             if (O < target_waves / 2) P = std::max(1LL, std::min((target_waves + O - 1) / O, (RG + 255) / 256));
@@ -1197,8 +1281,10 @@ namespace ormi::hip {
                 // UNR groups per lane starting at rg, 64 groups apart.
                 auto emit_step = [&](int UNR, const std::string& ind) {
                     g.declare_leaf_regs(b, ind, UNR);
+                    if (g.tail) b << ind << t << " pu_[" << UNR << "];\n";
                     b << ind << "#pragma unroll\n" << ind << "for (int u = 0; u < " << UNR << "; ++u) {\n";
                     b << ind << "  const " << t << " rgu = rg + u * 64;\n";
+                    if (g.tail) b << ind << "  pu_[u] = " << g.group_start("rgu") << ";\n";
                     g.declare_coords(b, ind + "  ", rd);
                     g.decompose(b, ind + "  ", "rgu", rd);
                     for (size_t L = 0; L < expr.leaves.size(); ++L) {
@@ -1211,8 +1297,12 @@ namespace ormi::hip {
                     b << ind << "#pragma unroll\n" << ind << "for (int u = 0; u < " << UNR << "; ++u) {\n";
                     b << ind << "#pragma unroll\n" << ind << "  for (int k = 0; k < " << V << "; ++k) {\n";
                     const std::string v = g.eval(b, ind + "    ", "u", "k");
-                    if (is_sum) b << ind << "    acc[k] += " << v << ";\n";
-                    else b << ind << "    ormi_am_step(mv[k], mi[k], " << v << ", (int)((rg + u * 64) * " << V << " + k));\n";
+                    // A ragged row's last group repeats elements of the one before:
+                    // a sum skips them, a maximum may take them twice.
+                    if (is_sum && g.tail) b << ind << "    if (pu_[u] + k >= (rg + u * 64) * " << V << ") acc[k] += " << v << ";\n";
+                    else if (is_sum) b << ind << "    acc[k] += " << v << ";\n";
+                    else b << ind << "    ormi_am_step(mv[k], mi[k], " << v << ", (int)("
+                           << (g.tail ? std::string("pu_[u]") : "(rg + u * 64) * " + std::to_string(V)) << " + k));\n";
                     b << ind << "  }\n" << ind << "}\n";
                 };
                 b << "  " << t << " rg = rg0 + lane;\n";
@@ -1242,8 +1332,8 @@ namespace ormi::hip {
                     // A non-empty chain of only -inf still holds the empty marker: its first
                     // element is the first maximum. An empty chain keeps the marker, an
                     // index above every real one (R < 2^31), so it loses every tie.
-                    b << "#pragma unroll\n  for (int k = 0; k < " << V << "; ++k) if (mi[k] == 0x7fffffff && rg0 + lane < rg1) mi[k] = (int)((rg0 + lane) * "
-                      << V << " + k);\n";
+                    b << "#pragma unroll\n  for (int k = 0; k < " << V << "; ++k) if (mi[k] == 0x7fffffff && rg0 + lane < rg1) mi[k] = (int)("
+                      << (V > 1 ? g.group_start("rg0 + lane") : std::string("rg0 + lane")) << " + k);\n";
                     b << "  float bv = mv[0]; int bi = mi[0];\n";
                     b << "#pragma unroll\n  for (int k = 1; k < " << V << "; ++k) ormi_am_take(bv, bi, mv[k], mi[k]);\n";
                     b << "  ormi_wave_argmax(bv, bi);\n";
@@ -1316,7 +1406,7 @@ namespace ormi::hip {
         // (each lane V consecutive columns, so a row segment is WC KB at V = 4)
         // and WR interleaved along the reduced rows. Fewer column waves when
         // the kept extent is narrow.
-        const long long IG = I / V;
+        const long long IG = (I + V - 1) / V;
         int WC = 1;
         while (WC * 2 <= std::min(tn.col_cwaves, tn.col_waves) && WC * 64LL < IG) WC *= 2;
         const int WR = std::max(1, tn.col_waves / WC);
@@ -1417,7 +1507,7 @@ namespace ormi::hip {
             else b << " sv[w][cl][k] = bv[k]; si[w][cl][k] = bx[k]; }\n";
             b << "  __syncthreads();\n";
             b << "  if (w == 0 && active) {\n";
-            b << "    const " << t << " e0 = (p * (" << t << ")NO + o) * (" << t << ")NI + ig * " << V << ";\n";
+            b << "    const " << t << " e0 = (p * (" << t << ")NO + o) * (" << t << ")NI + " << g.group_start("ig") << ";\n";
             b << "#pragma unroll\n    for (int k = 0; k < " << V << "; ++k) {\n";
             if (is_sum) {
                 b << "      float s = sv[0][cl][k];\n";

@@ -102,6 +102,11 @@ namespace ormi::hip {
             x.map_row_tile_wg_per_cu = std::clamp(env_int("ORMI_MAP_ROW_TILE_WG_PER_CU", x.map_row_tile_wg_per_cu), 0, 32);
             x.row_wg_per_cu = std::clamp(env_int("ORMI_ROW_WG_PER_CU", x.row_wg_per_cu), 0, 32);
             x.row_max_wg_per_cu = std::clamp(env_int("ORMI_ROW_MAX_WG_PER_CU", x.row_max_wg_per_cu), 0, 32);
+            x.rows_wg_per_cu = std::clamp(env_int("ORMI_ROWS_WG_PER_CU", x.rows_wg_per_cu), 1, 4096);
+            x.rows_regs = std::clamp(env_int("ORMI_ROWS_REGS", x.rows_regs), 16, 256);
+            x.rows_groups = std::clamp(env_int("ORMI_ROWS_GROUPS", x.rows_groups), 1, 32);
+            x.rows_col_block = std::clamp(env_int("ORMI_ROWS_COL_BLOCK", x.rows_col_block) / 256 * 256, 256, 1024);
+            x.rows_col_wg_per_cu = std::clamp(env_int("ORMI_ROWS_COL_WG_PER_CU", x.rows_col_wg_per_cu), 1, 64);
             x.map_nt_loads = env_int("ORMI_MAP_NT_LOADS", x.map_nt_loads) != 0;
             x.reduce_nt_loads = env_int("ORMI_REDUCE_NT_LOADS", x.reduce_nt_loads) != 0;
             x.nt_min_bytes = std::max(0, env_int("ORMI_NT_MIN_MIB", (int)(x.nt_min_bytes >> 20))) * (1LL << 20);
@@ -1594,6 +1599,502 @@ namespace ormi::hip {
         return plan;
     }
 
+    // ------------------------------------------------------- row programs --
+    namespace {
+        constexpr int kRowMaxWaves = 16;
+
+        // C expression of one element-wise instruction over named operands.
+        std::string lower_inst(const Inst& in, const std::vector<std::string>& name) {
+            if (in.op == OpEnum::CAST) {
+                if (in.cast == DType::BFloat16) return "ormi_round_bf16(" + name[in.a] + ")";
+                if (in.cast == DType::Float16) return "ormi_round_f16(" + name[in.a] + ")";
+                return name[in.a];
+            }
+            std::vector<std::string> operands{name[in.a]};
+            if (in.b >= 0) operands.push_back(name[in.b]);
+            if (!in.lower)
+                throw std::runtime_error(std::string("HIP JIT Compiler Error: No lowering rule registered for ") + ops::op_name(in.op));
+            return (*in.lower)(operands);
+        }
+        bool is_reduce_op(OpEnum op) { return op == OpEnum::SUM || op == OpEnum::MAX || op == OpEnum::ARGMAX; }
+    }  // namespace
+
+    // Lanes of a row: LPR lanes of one wave (several rows per wave) for rows of
+    // up to 64 lanes x U groups, else WR whole waves; each lane holds U groups
+    // of V elements of every per-element operand in registers. Stage s computes the
+    // per-row values that depend on s earlier reductions, then every reduction of
+    // values known by then, across the lanes (and through LDS across the
+    // waves) so that each lane has the result for the next stage; the outputs
+    // come last. With column sums, few work-groups walk the rows with a grid
+    // stride and accumulate the columns in registers over all their rows;
+    // without, every work-group takes one set of rows (on 16384 x 8192, row
+    // maximum, softmax denominator, mean and argmax: 77 us that way, 87-92 with
+    // 4-16 work-groups per compute unit walking the rows).
+    //
+    // What bounds it: HBM for long rows (those four statistics take the time of
+    // one read, 77-82 us, and 97 + 5.6 with the column sums, where the five
+    // separate kernels took 400), the arithmetic and the exchanges across the
+    // lanes for short ones (50021 x 301: 16 + 5 us, separately 81). Softmax of
+    // 16384 x 8192: 335 -> 175-185 us; a normalization's forward and backward
+    // over 4095 x 1536: 120 -> 26 us.
+    static bool plan_rows_uncached(const RowProgram& prog, int cu, RowPlan* plan) {
+        const Expr& expr = prog.expr;
+        const size_t nl = expr.leaves.size(), ni = expr.insts.size(), nout = prog.outs.size();
+        if (nout != expr.roots.size() || nout != prog.out_dtypes.size() || nout != prog.out_kinds.size() || !nout)
+            throw std::runtime_error("HIP codegen: one output buffer, dtype and kind per root.");
+        const Tuning& tn = tuning();
+        Gen g(expr);
+        g.out_dtypes = prog.out_dtypes;
+        g.want_off32 = tn.map_off32;
+        const int nd = (int)prog.shape.size();
+        for (int d = 0; d < nd; ++d) g.c.dims.push_back({(long long)prog.shape[d], d < nd - prog.reduced ? G_O : G_R});
+        for (const auto& L : expr.leaves) g.c.st.push_back(L.st);
+        canonicalize(g.c, g.scalar);
+        const long long O = group_size(g.c, G_O), R = group_size(g.c, G_R);
+        const std::vector<int> od = dims_of(g.c, G_O), rd = dims_of(g.c, G_R);
+        if (O < 2 || R < 2 || rd.size() != 1 || od.empty()) return false;
+        const int vd = rd[0];
+
+        // Value classes and levels.
+        std::vector<bool> row(nl + ni, false);
+        std::vector<int> level(nl + ni, 0);
+        int last_level = 0;
+        for (size_t L = 0; L < nl; ++L) row[L] = g.scalar[L] || g.c.st[L][vd] == 0;
+        for (size_t i = 0; i < ni; ++i) {
+            const Inst& in = expr.insts[i];
+            const size_t id = nl + i;
+            if (is_reduce_op(in.op)) {
+                row[id] = true;
+                level[id] = level[in.a] + (in.op == OpEnum::ARGMAX ? 2 : 1);
+            } else {
+                row[id] = row[in.a] && (in.b < 0 || row[in.b]);
+                level[id] = std::max(level[in.a], in.b < 0 ? 0 : level[in.b]);
+            }
+            last_level = std::max(last_level, level[id]);
+        }
+        // Operands held per element: those that vary along the row.
+        std::vector<size_t> held;
+        for (size_t L = 0; L < nl; ++L)
+            if (!row[L]) held.push_back(L);
+        if (held.empty()) return false;
+        size_t ncol = 0;
+        for (size_t r = 0; r < nout; ++r) {
+            if (prog.out_kinds[r] == RowOut::Column) ++ncol;
+            if (prog.out_kinds[r] == RowOut::Row && !row[expr.roots[r]]) throw std::runtime_error("HIP codegen: not a per-row value.");
+        }
+
+        bool vec_outs = true;
+        for (size_t r = 0; r < nout; ++r)
+            if (prog.out_kinds[r] == RowOut::Full) vec_outs = vec_outs && vector_dtype(prog.out_dtypes[r]);
+        g.choose_vec(vec_outs ? vd : -1, true);
+        g.vec_dim = vd;
+        const int V = g.vec;
+        const long long RG = g.groups(vd);
+        // Lanes per row and groups per lane.
+        const long long umax = std::max(1LL, std::min((long long)tn.rows_groups, (long long)tn.rows_regs / (V * (long long)(held.size() + ncol))));
+        int LPR = 64, WR = 1;
+        if (RG <= 64 * umax) {
+            // The fewest lanes that hold the row in umax groups each leave the
+            // fewest idle lanes and cross-lane steps, but a wave needs rows
+            // enough: no more rows per wave than leave two waves per SIMD.
+            LPR = 1;
+            while (LPR < 64 && (LPR * umax < RG || O * LPR < 64LL * 8 * std::max(cu, 1))) LPR *= 2;
+            while (LPR > 1 && LPR / 2 >= RG) LPR /= 2;
+        } else {
+            while (WR <= kRowMaxWaves && 64LL * WR * umax < RG) WR *= 2;
+            if (WR > kRowMaxWaves) return false;
+            // Few long rows: more waves share each, down to one group per lane.
+            while (WR < kRowMaxWaves && O * WR < 4LL * std::max(cu, 1) && 64LL * WR < RG) WR *= 2;
+        }
+        const int T = WR > 1 ? 64 * WR : LPR;  // lanes per row
+        const int U = (int)((RG + T - 1) / T);
+        const int block = std::max(ncol ? tn.rows_col_block : 256, T);
+        const int RPB = block / T;  // rows a work-group holds at once
+        const bool even = RG == (long long)T * U && !g.tail;
+
+        g.out_unaligned.assign(nout, false);
+        int out_bytes = 1;
+        for (size_t r = 0; r < nout; ++r) {
+            if (prog.out_kinds[r] != RowOut::Full) continue;
+            g.out_unaligned[r] = V > 1 && (R % 4 != 0 || ((uintptr_t)prog.outs[r] % 16) != 0);
+            out_bytes = std::max(out_bytes, (int)dtype_size(prog.out_dtypes[r]));
+        }
+        g.choose_nt_loads(tn.reduce_nt_loads, O * R);
+        const long long units = (O + RPB - 1) / RPB;
+        const int wg = ncol ? tn.rows_col_wg_per_cu : std::max(1, tn.rows_wg_per_cu * 256 / block);
+        const long long grid = std::min(units, (long long)std::max(cu, 1) * wg);
+        g.choose_idx(O * R + (grid + 1) * RPB, out_bytes);
+
+        KernelLaunch& k = plan->first;
+        plan->two_pass = ncol > 0;
+        plan->workspace_bytes = ncol * (size_t)grid * (size_t)R * sizeof(float);
+        if (ncol) g.args.ptr(false, "float", "part", nullptr);  // workspace bound later
+        for (size_t r = 0; r < nout; ++r)
+            if (prog.out_kinds[r] != RowOut::Column)
+                g.args.ptr(false, storage_type(prog.out_dtypes[r]), "out", prog.outs[r], (int)r);
+        g.declare_leaves();
+        g.args.i64("NO", O);
+        g.args.i64("NR", R);
+        g.args.i64("RG", RG);
+        g.declare_dims();
+        g.declare_strides();
+        k.grid[0] = (uint32_t)grid;
+        k.plan.kind = "rows";
+        for (auto [key, v] : {std::pair<const char*, long long>{"O", O}, {"R", R}, {"vec", V}, {"lanes", T}, {"groups", U},
+                              {"even", even ? 1 : 0}, {"idx", g.idx32 ? 32 : 64}, {"outputs", (long long)nout},
+                              {"columns", (long long)ncol}})
+            k.plan.add(key, v);
+        std::string layout = "|r";
+        for (int v : {T, WR, U, (int)even}) {
+            append_int(layout, v);
+            layout += ',';
+        }
+        for (RowOut x : prog.out_kinds) layout += char('0' + (int)x);
+
+        resolve(g, "rows", block, k, [&] {
+            const std::string t = g.idx();
+            std::ostringstream& b = g.body();
+            std::vector<std::string> name(nl + ni);
+            for (size_t L = 0; L < nl; ++L)
+                name[L] = g.scalar[L] ? "s" + std::to_string(L) : row[L] ? "y" + std::to_string(L) : "x" + std::to_string(L) + "[u][k]";
+            for (size_t i = 0; i < ni; ++i) name[nl + i] = (row[nl + i] ? "r" : "f") + std::to_string(i);
+            // Per-element instructions the values `need` depend on, in order.
+            auto closure = [&](const std::vector<int>& need) {
+                std::vector<bool> want(nl + ni, false);
+                for (int v : need) want[v] = true;
+                for (size_t i = ni; i-- > 0;) {
+                    const size_t id = nl + i;
+                    if (!want[id] || row[id]) continue;
+                    want[expr.insts[i].a] = true;
+                    if (expr.insts[i].b >= 0) want[expr.insts[i].b] = true;
+                }
+                std::vector<size_t> order;
+                for (size_t i = 0; i < ni; ++i)
+                    if (want[nl + i] && !row[nl + i]) order.push_back(i);
+                return order;
+            };
+            auto eval = [&](const std::string& ind, const std::vector<int>& need) {
+                for (size_t i : closure(need))
+                    b << ind << "const float " << name[nl + i] << " = " << lower_inst(expr.insts[i], name) << ";\n";
+            };
+            // Only a row's last groups can be past its end or repeat elements.
+            const std::string inside = even ? "true" : "(u < " + std::to_string(U - 1) + " || in_)";
+            const std::string counts = even ? "true"
+                                       : !g.tail ? inside
+                                                 : "(u < " + std::to_string(U - 1) + " || (in_ && p_[u] + k >= g_ * " + std::to_string(V) + "))";
+
+            g.hoist_scalars(b, "  ");
+            if (WR > 1) {
+                b << "  const int li = threadIdx.x % " << T << ", slot = threadIdx.x / " << T << ", wv = li >> 6, lane = li & 63;\n";
+            } else {
+                b << "  const int li = threadIdx.x % " << T << ", slot = threadIdx.x / " << T << ";\n";
+            }
+            // Group starts of this lane; the last group may lie past the row.
+            b << "  " << t << " p_[" << U << "];\n";
+            b << "  const " << t << " g_ = (" << t << ")(" << T * (U - 1) << " + li);\n";
+            b << "  const bool in_ = g_ < (" << t << ")RG;\n";
+            b << "#pragma unroll\n  for (int u = 0; u < " << U << "; ++u) {\n";
+            if (even) b << "    const " << t << " q_ = (" << t << ")(u * " << T << " + li);\n";
+            else b << "    const " << t << " q_ = u < " << U - 1 << " || in_ ? (" << t << ")(u * " << T << " + li) : (" << t << ")RG - 1;\n";
+            b << "    p_[u] = " << g.group_start("q_") << ";\n  }\n";
+            const std::string cv = "c" + std::to_string(vd);
+            std::vector<int> all = od;
+            all.push_back(vd);
+            std::vector<bool> across(nl, false);  // varies along the row only: read before the row loop
+            for (size_t L : held) {
+                across[L] = true;
+                for (int d : od) across[L] = across[L] && g.c.st[L][d] == 0;
+            }
+            // Operands that do not vary across rows are read once per work-group.
+            auto load_held = [&](const std::string& ind, bool before) {
+                for (size_t L : held)
+                    if (across[L] == before) b << ind << "float x" << L << "[" << U << "][" << V << "];\n";
+                b << "#pragma unroll\n" << ind << "for (int u = 0; u < " << U << "; ++u) {\n";
+                b << ind << "  const " << t << " " << cv << " = p_[u];\n";
+                for (size_t L : held) {
+                    if (across[L] != before) continue;
+                    const std::string off = g.offset(L, before ? rd : all);
+                    g.load_leaf(b, ind + "  ", L, off.empty() ? "0" : off, "x" + std::to_string(L) + "[u]");
+                }
+                b << ind << "}\n";
+            };
+            bool any_across = false;
+            for (size_t L : held) any_across = any_across || across[L];
+            if (any_across) load_held("  ", true);
+            // Column sums: one accumulator per element this lane holds.
+            std::vector<size_t> cols;
+            for (size_t r = 0; r < nout; ++r)
+                if (prog.out_kinds[r] == RowOut::Column) cols.push_back(r);
+            for (size_t j = 0; j < cols.size(); ++j)
+                b << "  float ca" << j << "[" << U << "][" << V << "];\n#pragma unroll\n  for (int u = 0; u < " << U
+                  << "; ++u)\n#pragma unroll\n    for (int k = 0; k < " << V << "; ++k) ca" << j << "[u][k] = 0.0f;\n";
+            // Reductions by the level they run at. An ARGMAX is the first index
+            // whose value equals the row's maximum, found at the level after
+            // that maximum (one the program may ask for besides): a compare and a
+            // select per element and an integer minimum across the lanes,
+            // where (value, index) pairs cost five operations per element and
+            // eight per exchange.
+            enum RedKind { kSum, kMax, kFirst };
+            struct Red {
+                RedKind kind;
+                int value;
+                std::vector<size_t> insts;
+                size_t id, of;  // of: the maximum a kFirst compares with
+            };
+            std::vector<std::vector<Red>> reds(last_level + 1);
+            size_t nred = 0;
+            auto red = [&](RedKind kind, int value, int lv, size_t of) -> Red& {
+                for (Red& x : reds[lv])
+                    if (x.kind == kind && x.value == value) return x;
+                reds[lv].push_back({kind, value, {}, nred++, of});
+                return reds[lv].back();
+            };
+            for (size_t i = 0; i < ni; ++i) {
+                const Inst& in = expr.insts[i];
+                if (!is_reduce_op(in.op)) continue;
+                if (in.op == OpEnum::SUM) red(kSum, in.a, level[in.a], 0).insts.push_back(i);
+                if (in.op == OpEnum::MAX) red(kMax, in.a, level[in.a], 0).insts.push_back(i);
+                if (in.op == OpEnum::ARGMAX) {
+                    const size_t m = red(kMax, in.a, level[in.a], 0).id;
+                    red(kFirst, in.a, level[in.a] + 1, m).insts.push_back(i);
+                }
+            }
+            if (WR > 1 && nred) {
+                // Alternate halves for alternate rows: a wave may start the next
+                // row while others still read this row's results.
+                b << "  __shared__ float rv_[2][" << nred << "][" << block / 64 << "];\n  int half = 0;\n";
+            }
+            b << "  for (" << t << " row0 = (" << t << ")blockIdx.x * " << RPB << "; row0 < (" << t << ")NO; row0 += (" << t << ")gridDim.x * " << RPB
+              << ") {\n";
+            b << "    const " << t << " row_ = row0 + (" << t << ")slot;\n";
+            if (RPB > 1) b << "    const bool live = row_ < (" << t << ")NO;\n    const " << t << " o = live ? row_ : (" << t << ")NO - 1;\n";
+            else b << "    const bool live = true;\n    const " << t << " o = row_;\n";
+            g.declare_coords(b, "    ", od);
+            g.decompose(b, "    ", "o", od);
+            load_held("    ", false);
+            for (size_t L = 0; L < nl; ++L) {
+                if (!row[L] || g.scalar[L]) continue;
+                const std::string off = g.offset(L, od);
+                const DType dt = expr.leaves[L].dtype;
+                const std::string p = "L" + std::to_string(L);
+                const std::string at = off.empty() ? "0" : off;
+                const std::string elem = g.off32 ? "*" + g.elem_ptr(std::string("const ") + storage_type(dt) + "*", p, at, dtype_size(dt), true)
+                                                 : p + "[" + at + "]";
+                b << "    const float y" << L << " = " << to_f32(dt, elem) << ";\n";
+            }
+            for (int lv = 0; lv <= last_level; ++lv) {
+                for (size_t i = 0; i < ni; ++i)
+                    if (row[nl + i] && level[nl + i] == lv && !is_reduce_op(expr.insts[i].op))
+                        b << "    const float " << name[nl + i] << " = " << lower_inst(expr.insts[i], name) << ";\n";
+                const auto& rs = reds[lv];
+                if (rs.empty()) continue;
+                // Sums and maxima share one pass over the lane's elements.
+                std::vector<int> need;
+                for (const Red& x : rs) {
+                    const std::string id = std::to_string(x.id);
+                    if (x.kind == kFirst) continue;
+                    need.push_back(x.value);
+                    b << "    float a" << id << "_[" << V << "];\n#pragma unroll\n    for (int k = 0; k < " << V << "; ++k) a" << id << "_[k] = "
+                      << (x.kind == kSum ? "0.0f" : "-__builtin_inff()") << ";\n";
+                }
+                if (!need.empty()) {
+                    b << "#pragma unroll\n    for (int u = 0; u < " << U << "; ++u) {\n#pragma unroll\n      for (int k = 0; k < " << V
+                      << "; ++k) {\n";
+                    eval("        ", need);
+                    for (const Red& x : rs) {
+                        const std::string id = std::to_string(x.id), v = name[x.value];
+                        if (x.kind == kSum) b << "        a" << id << "_[k] += " << (even ? v : counts + " ? " + v + " : 0.0f") << ";\n";
+                        if (x.kind == kMax)
+                            b << "        a" << id << "_[k] = ormi_maximum(a" << id << "_[k], "
+                              << (even ? v : inside + " ? " + v + " : -__builtin_inff()") << ");\n";
+                    }
+                    b << "      }\n    }\n";
+                }
+                for (const Red& x : rs) {
+                    if (x.kind != kFirst) continue;
+                    // Last group first, so the lane keeps its earliest hit. A
+                    // maximum is NaN when an element is: the first NaN then.
+                    const std::string id = std::to_string(x.id), v = name[x.value], m = "S" + std::to_string(x.of);
+                    b << "    int i" << id << "_[" << V << "];\n#pragma unroll\n    for (int k = 0; k < " << V << "; ++k) i" << id
+                      << "_[k] = 0x7fffffff;\n";
+                    for (const bool nan : {false, true}) {
+                        b << (nan ? "    else {\n" : "    if (" + m + " == " + m + ") {\n");
+                        b << "#pragma unroll\n      for (int u = " << U - 1 << "; u >= 0; --u) {\n#pragma unroll\n        for (int k = 0; k < " << V
+                          << "; ++k) {\n";
+                        eval("          ", {x.value});
+                        b << "          i" << id << "_[k] = " << (even ? std::string() : inside + " && ") << v
+                          << (nan ? " != " + v : " == " + m) << " ? (int)(p_[u] + k) : i" << id << "_[k];\n        }\n      }\n    }\n";
+                    }
+                }
+                for (const Red& x : rs) {
+                    const std::string id = std::to_string(x.id), lanes = "<" + std::to_string(std::min(T, 64)) + ">";
+                    const std::string a = (x.kind == kFirst ? "i" : "a") + id + "_";
+                    const std::string S = "S" + id;
+                    b << "    " << (x.kind == kFirst ? "int " : "float ") << S << " = ";
+                    if (V == 1) b << a << "[0];\n";
+                    else if (x.kind == kSum) b << "(" << a << "[0] + " << a << "[1]) + (" << a << "[2] + " << a << "[3]);\n";
+                    else {
+                        const std::string f = x.kind == kMax ? "ormi_maximum" : "min";
+                        b << f << "(" << f << "(" << a << "[0], " << a << "[1]), " << f << "(" << a << "[2], " << a << "[3]));\n";
+                    }
+                    b << "    " << S << " = " << (x.kind == kSum ? "ormi_lanes_sum" : x.kind == kMax ? "ormi_lanes_max" : "ormi_lanes_min")
+                      << lanes << "(" << S << ");\n";
+                    if (WR > 1)
+                        b << "    if (lane == 0) rv_[half][" << id << "][threadIdx.x >> 6] = "
+                          << (x.kind == kFirst ? "__int_as_float(" + S + ")" : S) << ";\n";
+                }
+                if (WR > 1) {
+                    b << "    __syncthreads();\n";
+                    for (const Red& x : rs) {
+                        const std::string id = std::to_string(x.id), S = "S" + id;
+                        auto at = [&](const std::string& w) {
+                            const std::string r = "rv_[half][" + id + "][slot * " + std::to_string(WR) + w + "]";
+                            return x.kind == kFirst ? "__float_as_int(" + r + ")" : r;
+                        };
+                        b << "    " << S << " = " << at("") << ";\n#pragma unroll\n    for (int w = 1; w < " << WR << "; ++w) ";
+                        if (x.kind == kSum) b << S << " += " << at(" + w") << ";\n";
+                        else b << S << " = " << (x.kind == kMax ? "ormi_maximum(" : "min(") << S << ", " << at(" + w") << ");\n";
+                    }
+                }
+                for (const Red& x : rs)
+                    for (size_t i : x.insts)
+                        b << "    const " << (x.kind == kFirst ? "int " : "float ") << name[nl + i] << " = S" << x.id << ";\n";
+            }
+            // Outputs.
+            std::vector<int> need;
+            std::vector<size_t> full;
+            for (size_t r = 0; r < nout; ++r) {
+                if (prog.out_kinds[r] == RowOut::Full) full.push_back(r);
+                if (prog.out_kinds[r] != RowOut::Row) need.push_back(expr.roots[r]);
+            }
+            if (!need.empty()) {
+                b << "#pragma unroll\n    for (int u = 0; u < " << U << "; ++u) {\n";
+                for (size_t r : full) b << "      float w" << r << "[" << V << "];\n";
+                b << "#pragma unroll\n      for (int k = 0; k < " << V << "; ++k) {\n";
+                eval("        ", need);
+                for (size_t r : full) b << "        w" << r << "[k] = " << name[expr.roots[r]] << ";\n";
+                for (size_t j = 0; j < cols.size(); ++j) {
+                    const std::string v = name[expr.roots[cols[j]]];
+                    const std::string live = RPB > 1 ? (even ? std::string("live") : "live && " + counts) : counts;
+                    if (live == "true") b << "        ca" << j << "[u][k] += " << v << ";\n";
+                    else b << "        ca" << j << "[u][k] += " << live << " ? " << v << " : 0.0f;\n";
+                }
+                b << "      }\n";
+                if (!full.empty()) {
+                    b << "      if (live && " << inside << ") {\n";
+                    b << "        const " << t << " eo = o * (" << t << ")NR + p_[u];\n";
+                    for (size_t r : full) {
+                        const DType odt = prog.out_dtypes[r];
+                        const std::string on = "out" + std::to_string(r);
+                        if (V == 4) {
+                            const std::string vt = g.group_type(odt, g.out_unaligned[r]);
+                            std::string val = g.group_type(odt, false) + "{";
+                            for (int q = 0; q < 4; ++q)
+                                val += (q ? ", " : "") + from_f32(odt, "w" + std::to_string(r) + "[" + std::to_string(q) + "]");
+                            val += "}";
+                            const std::string addr = g.elem_ptr(vt + "*", on, "eo", dtype_size(odt), false);
+                            if (tn.map_nt_stores) b << "        __builtin_nontemporal_store(" << val << ", " << addr << ");\n";
+                            else b << "        *" << addr << " = " << val << ";\n";
+                        } else {
+                            b << "        *" << g.elem_ptr(std::string(storage_type(odt)) + "*", on, "eo", dtype_size(odt), false) << " = "
+                              << from_f32(odt, "w" + std::to_string(r) + "[0]") << ";\n";
+                        }
+                    }
+                    b << "      }\n";
+                }
+                b << "    }\n";
+            }
+            bool any_row = false;
+            for (size_t r = 0; r < nout; ++r) any_row = any_row || prog.out_kinds[r] == RowOut::Row;
+            if (any_row) {
+                b << "    if (li == 0 && live) {\n";
+                for (size_t r = 0; r < nout; ++r) {
+                    if (prog.out_kinds[r] != RowOut::Row) continue;
+                    const int v = expr.roots[r];
+                    const bool arg = (size_t)v >= nl && expr.insts[v - nl].op == OpEnum::ARGMAX;
+                    b << "      out" << r << "[o] = " << (arg ? "(long long)" + name[v] : from_f32(prog.out_dtypes[r], name[v])) << ";\n";
+                }
+                b << "    }\n";
+            }
+            if (WR > 1 && nred) b << "    half ^= 1;\n";
+            b << "  }\n";
+            if (!cols.empty()) {
+                // The work-group's rows of lanes: those of one wave combine by
+                // lane exchanges, its RPB sets through LDS in slot order.
+                const int sets = WR > 1 ? RPB : block / 64;
+                for (size_t j = 0; j < cols.size(); ++j) {
+                    b << "#pragma unroll\n  for (int u = 0; u < " << U << "; ++u)\n#pragma unroll\n    for (int k = 0; k < " << V << "; ++k) {\n";
+                    if (WR == 1)
+                        for (int x = T; x < 64; x *= 2) b << "      ca" << j << "[u][k] += __shfl_xor(ca" << j << "[u][k], " << x << ", 64);\n";
+                    b << "    }\n";
+                }
+                if (sets > 1) b << "  __shared__ float cs_[" << sets << "][" << T << "][" << V << "];\n";
+                const std::string set = WR > 1 ? "slot" : "(int)(threadIdx.x >> 6)";
+                const std::string first = WR > 1 ? "true" : "(int)(threadIdx.x & 63) < " + std::to_string(T);
+                for (size_t j = 0; j < cols.size(); ++j) {
+                    b << "#pragma unroll\n  for (int u = 0; u < " << U << "; ++u) {\n";
+                    if (sets > 1) {
+                        b << "    __syncthreads();\n";
+                        b << "    if (" << first << ") for (int k = 0; k < " << V << "; ++k) cs_[" << set << "][li][k] = ca" << j << "[u][k];\n";
+                        b << "    __syncthreads();\n";
+                        b << "    if (threadIdx.x < " << T << ")\n#pragma unroll\n      for (int k = 0; k < " << V
+                          << "; ++k) { float s = cs_[0][li][k]; for (int w = 1; w < " << sets << "; ++w) s += cs_[w][li][k]; ca" << j
+                          << "[u][k] = s; }\n";
+                    }
+                    const std::string in_row = even ? "" : " && " + inside;
+                    b << "    if (threadIdx.x < " << T << in_row << ") {\n";
+                    // A ragged row's repeated elements belong to the group before.
+                    b << "#pragma unroll\n      for (int k = 0; k < " << V << "; ++k) if (" << counts << ") part[((long long)" << j
+                      << " * gridDim.x + blockIdx.x) * NR + p_[u] + k] = ca" << j << "[u][k];\n";
+                    b << "    }\n  }\n";
+                }
+            }
+        }, layout);
+        if (!ncol) return true;
+
+        // Column sums of the work-groups: 16 waves per 64 columns walk the parts
+        // with a stride of 16, 16 loads in flight, and the first wave adds
+        // the 16 runs in wave order.
+        KernelLaunch& s2 = plan->second;
+        Gen g2(no_expr());
+        g2.args.ptr(true, "float", "part", nullptr);
+        int j2 = 0;
+        for (size_t r = 0; r < nout; ++r)
+            if (prog.out_kinds[r] == RowOut::Column) {
+                g2.args.ptr(false, "float", "out", prog.outs[r], (int)r);
+                ++j2;
+            }
+        g2.args.i64("NR", R);
+        g2.args.i64("NP", grid);
+        s2.grid[0] = (uint32_t)((R + 63) / 64);
+        s2.grid[1] = (uint32_t)ncol;
+        s2.plan.kind = "rows-columns";
+        std::string which = "|c";
+        for (size_t r = 0; r < nout; ++r)
+            if (prog.out_kinds[r] == RowOut::Column) {
+                append_int(which, (long long)r);
+                which += ',';
+            }
+        resolve(g2, "rowscol", 1024, s2, [&] {
+            std::ostringstream& b = g2.body();
+            b << "  __shared__ float v_[16][64];\n";
+            b << "  const int c = threadIdx.x & 63, q = threadIdx.x >> 6;\n";
+            b << "  const long long e = (long long)blockIdx.x * 64 + c;\n";
+            b << "  const long long ec = e < NR ? e : NR - 1;\n";
+            b << "  const float* src = part + (long long)blockIdx.y * NP * NR + ec;\n";
+            b << "  float s = 0.0f;\n  for (long long p0 = q; p0 < NP; p0 += 256) {\n    float v[16];\n";
+            b << "#pragma unroll\n    for (int j = 0; j < 16; ++j) v[j] = p0 + 16 * j < NP ? src[(p0 + 16 * j) * NR] : 0.0f;\n";
+            b << "#pragma unroll\n    for (int j = 0; j < 16; ++j) s += v[j];\n  }\n";
+            b << "  v_[q][c] = s;\n  __syncthreads();\n";
+            b << "  if (q != 0 || e >= NR) return;\n";
+            b << "  for (int w = 1; w < 16; ++w) s += v_[w][c];\n";
+            int j = 0;
+            for (size_t r = 0; r < nout; ++r)
+                if (prog.out_kinds[r] == RowOut::Column) b << "  if (blockIdx.y == " << j++ << ") out" << r << "[e] = s;\n";
+        }, which);
+        return true;
+    }
+
     // Point the split-reduction kernels at the workspace: values first, then
     // indices. The first kernel's outp/outi are args 0 and 1; the second
     // kernel's pvals/pidx are args 1 and 2.
@@ -1628,6 +2129,7 @@ namespace ormi::hip {
             std::mutex mu;
             std::unordered_map<std::string, KernelLaunch> maps;
             std::unordered_map<std::string, ReducePlan> reduces;
+            std::unordered_map<std::string, RowPlan> rows;  // a declined program has no kernel name
         };
         RequestCache& request_cache() {
             static auto* c = new RequestCache();
@@ -1742,6 +2244,46 @@ namespace ormi::hip {
         if (rc.reduces.size() >= kMaxRequests) rc.reduces.clear();
         rc.reduces.emplace(std::move(kb.s), plan);
         return plan;
+    }
+
+    bool plan_rows(const RowProgram& p, int cu, RowPlan* plan, bool launch_only) {
+        KeyBuf kb;
+        kb.i64('P');
+        kb.i64(cu);
+        kb.i64((long long)p.shape.size() | ((long long)p.reduced << 8));
+        for (int d : p.shape) kb.i64(d);
+        for (size_t r = 0; r < p.outs.size(); ++r)
+            kb.i64((long long)p.out_dtypes[r] | ((long long)p.out_kinds[r] << 8) | ((long long)((uintptr_t)p.outs[r] & 255) << 16));
+        key_expr(kb, p.expr);
+        RequestCache& rc = request_cache();
+        auto use = [&](RowPlan& c) {
+            if (c.first.args.empty()) return false;
+            refresh_handle(c.first);
+            plan->two_pass = c.two_pass;
+            plan->workspace_bytes = c.workspace_bytes;
+            plan->first = instantiate(c.first, p.expr, p.outs.data(), launch_only);
+            if (c.two_pass) {
+                refresh_handle(c.second);
+                plan->second = instantiate(c.second, p.expr, p.outs.data(), launch_only);
+            }
+            return true;
+        };
+        {
+            std::lock_guard<std::mutex> lock(rc.mu);
+            auto it = rc.rows.find(kb.s);
+            if (it != rc.rows.end()) return use(it->second);
+        }
+        RowPlan made;
+        if (!plan_rows_uncached(p, cu, &made)) made = RowPlan{};
+        std::lock_guard<std::mutex> lock(rc.mu);
+        if (rc.rows.size() >= kMaxRequests) rc.rows.clear();
+        return use(rc.rows.emplace(std::move(kb.s), std::move(made)).first->second);
+    }
+
+    // The partial column sums are the first argument of both kernels.
+    void bind_rows_workspace(RowPlan& plan, void* ws) {
+        if (!plan.two_pass) return;
+        plan.first.args[0] = plan.second.args[0] = (uint64_t)(uintptr_t)ws;
     }
 
     void bind_workspace(ReducePlan& plan, void* ws) {

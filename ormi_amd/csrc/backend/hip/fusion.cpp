@@ -153,7 +153,7 @@ namespace ormi::hip {
         return interior;
     }
 
-    static Leaf make_leaf(const NodePtr& n, const std::vector<int>& shape, bool plan_only) {
+    Leaf make_leaf(const NodePtr& n, const std::vector<int>& shape, bool plan_only) {
         if (!n->data) throw std::runtime_error("HIP codegen: leaf is not realized.");
         if (!plan_only && n->device.type != DeviceEnum::HIP) throw std::runtime_error("HIP codegen: operand lives on another device.");
         Leaf L;

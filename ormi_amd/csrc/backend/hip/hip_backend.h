@@ -53,6 +53,24 @@ namespace ormi::hip {
     // shape), else nullptr. The scheduler then realizes both with one kernel.
     NodePtr epilogue_reduction(const NodePtr& n);
 
+    // n (realized, or with a host stand-in buffer when plan_only) as a leaf of a kernel
+    // over `shape`: its strides right-aligned, 0 where it broadcasts.
+    Leaf make_leaf(const NodePtr& n, const std::vector<int>& shape, bool plan_only = false);
+
+    // ---------------------------------------------------- row programs --
+    // Whether realizing root runs as a row program (rows.cpp), and the
+    // unrealized nodes that one reads.
+    bool row_program_frontier(const NodePtr& root, std::vector<NodePtr>* frontier);
+    // The kernels that realizing `roots` together as one row program would
+    // launch (planning only: operands may live on any device); false when they
+    // are none.
+    bool plan_row_program(const std::vector<NodePtr>& roots, int compute_units, RowPlan* plan);
+    // Realizes root (and the reductions it reads) as one; false when it is none.
+    bool run_row_program(const NodePtr& root);
+    // Realizes those of `roots` that share operands in row programs; the others
+    // stay unrealized.
+    void realize_row_groups(const std::vector<NodePtr>& roots);
+
     // ------------------------------------------------------- scheduler --
     // Realize root on the HIP device: pointwise regions become one fused
     // kernel, reductions fuse their pointwise producer as a prologue, views

@@ -124,6 +124,18 @@ namespace ormi::hip {
         // Both load hints apply only to leaves read once (no broadcast), in
         // kernels whose such leaves bring in at least this many bytes.
         long long nt_min_bytes = 64LL << 20;
+        int rows_wg_per_cu = 4096;       // work-groups per CU that walk the rows of a row program
+        // Row programs. Registers per lane for held operands and column sums, at
+        // most rows_groups groups of each. Work-groups per compute unit without
+        // column sums (no limit in practice) and with them: every work-group then
+        // leaves one partial row, and 3 measured best on 16384 x 8192 (row
+        // kernel + finish: 2: 109 + 6.0, 3: 97 + 8.7, 4: 101 + 11.1, 5: 109 + 13.6
+        // us with the first finish kernel; 512 threads, 2: 111 + 5.9).
+        int rows_regs = 128;
+        int rows_groups = 8;
+        int rows_wg_per_cu = 4096;
+        int rows_col_wg_per_cu = 3;
+        int rows_col_block = 256;
         bool map_off32 = true;        // 32-bit byte offsets from uniform bases when they fit (map)
         bool map_rows = true;         // row-aligned tiles when a tile covers whole rows or lies in one (map)
         bool map_row_tiles = true;    // tiles of `unroll` rows x 256 groups when an operand is a bias row (map)
@@ -165,6 +177,35 @@ namespace ormi::hip {
     };
     ReducePlan plan_reduce(const Expr& expr, const std::vector<int>& in_shape, const std::vector<int>& axes, ReduceOp op,
                            void* out, int compute_units, bool launch_only = false, const StoreEpilogue* epilogue = nullptr);
+    // A row program: several reductions over the same trailing dims of one
+    // shape, and element-wise values over that shape or over its rows, as one
+    // kernel that reads each operand once and keeps a row in registers from
+    // one stage to the next. expr.insts may hold SUM, MAX and ARGMAX (of
+    // operand a, over the last `reduced` dims) besides element-wise ops; a
+    // value is either one per element or one per row (a reduction, an operand
+    // that does not vary along a row, or an op of such values), and a per-row
+    // value reads as a constant along its row. One output per expr.roots
+    // entry: a contiguous buffer of the shape (Full), of one value per row (Row; an
+    // ARGMAX as int64), or the fp32 sum of a per-element value over the rows, one per
+    // element of a row (Column). An ARGMAX is an output only, never an operand.
+    enum class RowOut { Full, Row, Column };
+    struct RowProgram {
+        Expr expr;
+        std::vector<int> shape;
+        int reduced = 1;
+        std::vector<void*> outs;
+        std::vector<DType> out_dtypes;
+        std::vector<RowOut> out_kinds;
+    };
+    // two_pass (column outputs): `second` combines the work-groups' column
+    // sums, which go to a workspace.
+    using RowPlan = ReducePlan;
+    // False when the generator has no row kernel for it: fewer than two rows or
+    // elements per row, rows too long for the registers, a layout whose reduced
+    // dims do not merge. Otherwise *plan is the launch.
+    bool plan_rows(const RowProgram& p, int compute_units, RowPlan* plan, bool launch_only = false);
+    void bind_rows_workspace(RowPlan& plan, void* workspace);
+
     // Generated kernels launched by this process so far (tests count fusions).
     unsigned long long kernel_launches();
     void bind_workspace(ReducePlan& plan, void* workspace);

@@ -656,8 +656,16 @@ namespace ormi::hip {
         launch(plan_map(e, root->view.shape, out->ptr, root->dtype, device_compute_units(), true));
     }
 
-    // Nodes that must hold buffers before `n` can run as one step: a view's
-    // parent, an element-wise region's frontier, the frontier (or the input)
+    // Whether a region with this frontier may be part of a row program: it
+    // reads a reduction, or a broadcast or reshaped one, that has no buffer yet.
+    static bool reads_a_reduction(const std::vector<NodePtr>& front) {
+        for (const auto& f : front)
+            if (!f->is_realized() && (is_view_op(f->op) || ops::is_reduction(f->op))) return true;
+        return false;
+    }
+
+    // Nodes that must hold buffers before `n` can run as one step: a row
+    // program's leaves, a view's parent, an element-wise region's frontier, the frontier (or the input)
     // of a reduction, a matmul's operands.
     static std::vector<NodePtr> dependencies(const NodePtr& n) {
         if (is_view_op(n->op)) return {n->parents[0]};
@@ -670,11 +678,17 @@ namespace ormi::hip {
                 return deps;
             }
             if (const NodePtr r = epilogue_reduction(n)) return dependencies(r);
-            return region_frontier(n);
+            std::vector<NodePtr> front = region_frontier(n);
+            if (reads_a_reduction(front)) row_program_frontier(n, &front);
+            return front;
         }
         if (ops::is_reduction(n->op)) {
             const NodePtr& x = n->parents[0];
-            if (fuse_as_prologue(x)) return region_frontier(x);
+            if (fuse_as_prologue(x)) {
+                std::vector<NodePtr> front = region_frontier(x);
+                if (reads_a_reduction(front)) row_program_frontier(n, &front);
+                return front;
+            }
             return {x};
         }
         return n->parents;
@@ -688,9 +702,14 @@ namespace ormi::hip {
             return;
         }
         if (fusible_root(*n)) {
+            EpilogueMatch m;
+            if (!match_epilogue(n, m) && !epilogue_reduction(n) && reads_a_reduction(region_frontier(n)) && run_row_program(n)) return;
             run_map(n);
             return;
         }
+        if (ops::is_reduction(n->op) && fuse_as_prologue(n->parents[0]) && reads_a_reduction(region_frontier(n->parents[0])) &&
+            run_row_program(n))
+            return;
         if (n->op == OpEnum::MATMUL) {
             // Its operands are realized, and so are the activation's (the same).
             if (const NodePtr a = activation_consumer(n)) {
@@ -735,6 +754,17 @@ namespace ormi::hip {
 
     void realize_group(const std::vector<NodePtr>& roots) {
         ScopeGuard guard(roots.data(), roots.size());
+        for (const auto& r : roots)
+            if (r && !r->is_realized() && r->device.type != DeviceEnum::HIP)
+                throw std::runtime_error("HIP scheduler: node belongs to another device.");
+        {
+            std::vector<NodePtr> open;
+            for (const auto& r : roots) {
+                EpilogueMatch m;
+                if (r && !r->is_realized() && !match_epilogue(r, m)) open.push_back(r);
+            }
+            if (open.size() >= 2) realize_row_groups(open);
+        }
         // Element-wise roots with float results that can share one kernel,
         // grouped by shape in first-seen order; everything else realizes alone.
         std::vector<std::pair<std::vector<int>, std::vector<NodePtr>>> groups;

@@ -205,6 +205,23 @@ namespace {
         return d;
     }
 
+    // The kernels of the row program that realize_all would run for these
+    // nodes, or None when they are none (planning only).
+    py::object plan_rows_program(const std::vector<std::shared_ptr<Node>>& roots) {
+        hip::RowPlan rp;
+        if (!hip::plan_row_program(roots, 256, &rp)) return py::none();
+        py::dict d;
+        d["source"] = hip::kernel_source(rp.first);
+        d["name"] = rp.first.name;
+        d["plan"] = rp.first.plan.text();
+        d["grid"] = std::vector<uint32_t>{rp.first.grid[0], rp.first.grid[1], rp.first.grid[2]};
+        d["block"] = rp.first.block[0];
+        d["two_pass"] = rp.two_pass;
+        d["second_source"] = hip::kernel_source(rp.second);
+        d["workspace_bytes"] = rp.workspace_bytes;
+        return d;
+    }
+
     // The multi-output kernel realize_all would launch for these element-wise
     // roots of one shape (planning only: operands may live on any device).
     py::dict plan_group(const std::vector<std::shared_ptr<Node>>& roots) {
@@ -383,6 +400,7 @@ PYBIND11_MODULE(ormi_backend, m) {
           "Pairs of independent products the HIP scheduler ran as one grouped GEMM launch in this process.");
     m.def("_plan_kernel", &plan_kernel);
     m.def("_plan_group", &plan_group);
+    m.def("_plan_rows", &plan_rows_program);
     m.def("realize_all", &execute_graph_group,
           "Realize several nodes together; on the HIP device same-shape element-wise roots share one kernel.");
     m.def("_fastdiv", [](uint32_t d) {

@@ -214,3 +214,42 @@ __device__ __forceinline__ void ormi_wave_argmax(float& v, int& i) {
     ormi_am_take(v, i, __shfl_xor(v, 16, 64), __shfl_xor(i, 16, 64));
     ormi_am_take(v, i, __shfl_xor(v, 32, 64), __shfl_xor(i, 32, 64));
 }
+
+// The same over groups of N = 1, 2, 4, ..., 64 consecutive lanes: every lane
+// of a group ends with its group's result (N = 64: the orders above).
+template <int N>
+__device__ __forceinline__ float ormi_lanes_sum(float v) {
+    if (N >= 2) v += ormi_dpp_f<0xB1>(v);
+    if (N >= 4) v += ormi_dpp_f<0x4E>(v);
+    if (N >= 8) v += ormi_dpp_f<0x141>(v);
+    if (N >= 16) v += ormi_dpp_f<0x140>(v);
+    if (N >= 32) v += __shfl_xor(v, 16, 64);
+    if (N >= 64) v += __shfl_xor(v, 32, 64);
+    return v;
+}
+
+// The larger of two values, NaN when either is (IEEE 754-2019 maximum, +0 above
+// -0): one instruction on gfx950.
+__device__ __forceinline__ float ormi_maximum(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+
+template <int N>
+__device__ __forceinline__ float ormi_lanes_max(float v) {
+    if (N >= 2) v = ormi_maximum(v, ormi_dpp_f<0xB1>(v));
+    if (N >= 4) v = ormi_maximum(v, ormi_dpp_f<0x4E>(v));
+    if (N >= 8) v = ormi_maximum(v, ormi_dpp_f<0x141>(v));
+    if (N >= 16) v = ormi_maximum(v, ormi_dpp_f<0x140>(v));
+    if (N >= 32) v = ormi_maximum(v, __shfl_xor(v, 16, 64));
+    if (N >= 64) v = ormi_maximum(v, __shfl_xor(v, 32, 64));
+    return v;
+}
+
+template <int N>
+__device__ __forceinline__ int ormi_lanes_min(int v) {
+    if (N >= 2) v = min(v, ormi_dpp_i<0xB1>(v));
+    if (N >= 4) v = min(v, ormi_dpp_i<0x4E>(v));
+    if (N >= 8) v = min(v, ormi_dpp_i<0x141>(v));
+    if (N >= 16) v = min(v, ormi_dpp_i<0x140>(v));
+    if (N >= 32) v = min(v, __shfl_xor(v, 16, 64));
+    if (N >= 64) v = min(v, __shfl_xor(v, 32, 64));
+    return v;
+}

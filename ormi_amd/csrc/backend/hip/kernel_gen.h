@@ -124,7 +124,6 @@ namespace ormi::hip {
         // Both load hints apply only to leaves read once (no broadcast), in
         // kernels whose such leaves bring in at least this many bytes.
         long long nt_min_bytes = 64LL << 20;
-        int rows_wg_per_cu = 4096;       // work-groups per CU that walk the rows of a row program
         // Row programs. Registers per lane for held operands and column sums, at
         // most rows_groups groups of each. Work-groups per compute unit without
         // column sums (no limit in practice) and with them: every work-group then

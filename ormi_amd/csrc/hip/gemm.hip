@@ -1696,6 +1696,33 @@ static int gemm_packed_locked(const ormi_gemm_desc* d, const Epi& epi, long long
     return gemm_run_locked(&dp, epi, batch, false, true);
 }
 
+// Whether gemm_direct.hip's kernels take a product (both operands unit-stride
+// in one index). Measured against the kernels that would run otherwise, on
+// about 80 shapes from 1 x 1 x 5000 to 4095^3, operands rotating through memory:
+//   * operands in whole 16-byte chunks with K in whole k-tiles, where the
+//     direct-load tiles run: while those tiles number under a third (fp32: a
+//     quarter) of the compute units, up to 2^31 multiply-adds (1024^3 bf16
+//     17.6 -> 12.0 us, 512^3 8.8 -> 5.4, 12 x 8192 x 2048 15.1 -> 12.3; past the
+//     line 2048^3 26 against 59, 200 x 4096^2 22 against 44, fp32 1024^3 26.6
+//     against 25.7);
+//   * otherwise packing, the register-staged kernels or the generic one would
+//     run: up to 2.7e9 multiply-adds in 16 bits (1001 x 1003 x 1005 34.4 -> 20.2,
+//     6 x 1544 x 2648 25.8 -> 12.4, 1500^3 47 against 70 us) and 2^33 in fp32
+//     (2047 x 2049 x 1023 150 -> 113.5, 424 x 56 x 248 21.6 -> 6.0, 4095^2 x 1001
+//     280 against 330-409).
+// A forced configuration of the other kernels (their environment variables)
+// keeps them.
+static bool takes_direct(const ormi_gemm_desc* d, long long batch, bool fast) {
+    for (const char* forced : {"ORMI_GEMM_DMA_CFG", "ORMI_GEMM_F32_DMA_CFG", "ORMI_GEMM_CFG16", "ORMI_GEMM_CFG32", "ORMI_GEMM_DMA",
+                               "ORMI_GEMM_F32_DMA", "ORMI_GEMM_MAX_SPLITS", "ORMI_GEMM_PACK"})
+        if (std::getenv(forced)) return false;
+    const long long macs = batch * d->M * d->N * (long long)d->K;
+    const long long t128 = batch * ((d->M + 127) / 128) * ((d->N + 127) / 128);
+    const bool f32 = d->dtype == ORMI_DTYPE_F32;
+    if (fast && d->K % (f32 ? 32 : 64) == 0) return t128 < (f32 ? compute_units() / 4 : compute_units() / 3) && macs <= (1LL << 31);
+    return macs <= (f32 ? 1LL << 33 : 5LL << 29);
+}
+
 static int gemm_run_locked(const ormi_gemm_desc* d, const Epi& epi, long long batch, bool noalloc, bool packed) {
     int rc = ORMI_HIP_OK;
     auto workspace = [noalloc](size_t bytes, void** out) {
@@ -1754,6 +1781,25 @@ static int gemm_run_locked(const ormi_gemm_desc* d, const Epi& epi, long long ba
     }
 
     hipError_t e;
+    const int direct_env = env_cfg("ORMI_GEMM_DIRECT", 1);
+    if (direct_env != 0 && !packed && (a_kc || a_mc) && (b_kc || b_nc) && (direct_env == 2 || takes_direct(d, batch, fast))) {
+        const DirectPlan r = gemm_direct_plan(d, batch, a_kc, b_kc);
+        if (r.mt > 0) {
+            if (r.splits > 1) {
+                void* ws = nullptr;
+                rc = workspace((size_t)batch * d->M * d->N * r.splits * sizeof(float), &ws);
+                if (rc != ORMI_HIP_OK) return rc;
+                p.c = (float*)ws;
+                p.epi = Epi{};
+                p.epi.kind = ORMI_GEMM_EPI_NONE;
+            }
+            gemm_direct_launch(d, p, batch, r, a_kc, b_kc);
+            if (r.splits > 1) launch_finish(d, p.c, r.splits, batch, epi);
+            e = hipGetLastError();
+            if (e != hipSuccess) return fail(ORMI_HIP_ERR_RUNTIME, std::string("ormi_hip_gemm launch: ") + hipGetErrorString(e));
+            return ORMI_HIP_OK;
+        }
+    }
     // Operands the fast kernels cannot take are packed into dense k-contiguous
     // buffers first, unless the product is small (the generic kernel is then
     // at its launch floor anyway) or the caller cannot allocate.

@@ -573,4 +573,13 @@ void run32_dma_persist(const GemmParams& p, int groups, bool a_kc, bool b_kc);
 bool run32_dma_pair(const GemmParams& p0, bool a_kc0, bool b_kc0, const GemmParams& p1, bool a_kc1, bool b_kc1,
                     int groups);
 
+// Products by register fragments loaded straight from memory (gemm_direct.hip):
+// 16 mt x 16 nt tiles, one per work-group, whose `waves` split K. Operands have
+// a unit stride along k (kc) or along m / n, any alignment. mt = 0: not possible.
+struct DirectPlan {
+    int mt = 0, nt = 0, waves = 1, splits = 1;
+};
+DirectPlan gemm_direct_plan(const ormi_gemm_desc* d, long long batch, bool a_kc, bool b_kc);
+void gemm_direct_launch(const ormi_gemm_desc* d, GemmParams& p, long long batch, const DirectPlan& r, bool a_kc, bool b_kc);
+
 }  // namespace ormi_hip

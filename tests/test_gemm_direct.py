@@ -1,0 +1,186 @@
+"""Products by register fragments loaded straight from memory
+(gemm_direct.hip): the sizes where tiles, fragments and k-steps end (1, 15..17,
+31..33, 63..65 and the like), every pair of layouts and types, unaligned bases
+and row strides, K shares that leave waves without a step, splits across
+work-groups, batches with a broadcast operand, and every epilogue, in place too.
+
+Bound: the componentwise error of a length-K fp32 accumulation in any order, of
+products that are exact in fp32 for 16-bit operands and rounded once for fp32:
+(K + 2) eps32 (|A| |B|); an epilogue adds its own few roundings."""
+import ctypes
+
+import numpy as np
+import pytest
+from test_gemm_epilogue import Epi
+from test_map_cabi import Dev
+
+EPS32 = float(np.finfo(np.float32).eps)
+F32, BF16, F16 = 0, 3, 4
+
+
+class Desc(ctypes.Structure):
+    _fields_ = [("dtype", ctypes.c_int), ("M", ctypes.c_int), ("N", ctypes.c_int), ("K", ctypes.c_int),
+                ("a", ctypes.c_void_p), ("a_stride_m", ctypes.c_int64), ("a_stride_k", ctypes.c_int64),
+                ("b", ctypes.c_void_p), ("b_stride_k", ctypes.c_int64), ("b_stride_n", ctypes.c_int64),
+                ("c", ctypes.c_void_p), ("batch_ndim", ctypes.c_int), ("batch_shape", ctypes.c_int * 4),
+                ("a_batch_stride", ctypes.c_int64 * 4), ("b_batch_stride", ctypes.c_int64 * 4)]
+
+
+def storage(x, dtype):
+    """x's bits in dtype and the float64 values they hold."""
+    if dtype == F32:
+        return x, x.astype(np.float64)
+    if dtype == F16:
+        h = x.astype(np.float16)
+        return h, h.astype(np.float64)
+    u = x.view(np.uint32)
+    h = ((u + 0x7FFF + ((u >> 16) & 1)) >> 16).astype(np.uint16)
+    return h, (h.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+
+
+class Product:
+    """Operands in padded buffers (row pitch = extent + pad, base shifted by
+    `shift` elements) so that nothing but the element size is aligned."""
+
+    def __init__(self, lib, dtype, layout, M, N, K, batch=1, share_b=False, pad=0, shift=0, seed=0):
+        self.lib, self.dev, self.M, self.N, self.K, self.batch = lib, Dev(lib), M, N, K, batch
+        rng = np.random.default_rng(seed + M * 7 + N * 3 + K)
+        es = 4 if dtype == F32 else 2
+
+        def operand(rows, cols, count):
+            x = rng.standard_normal((count, rows, cols)).astype(np.float32)
+            bits, val = storage(x, dtype)
+            buf = np.zeros((count, rows, cols + pad), bits.dtype)
+            buf[:, :, :cols] = bits
+            raw = np.concatenate([np.zeros(shift, bits.dtype), buf.reshape(-1)])
+            p = self.dev.alloc(raw.nbytes)
+            assert lib.ormi_hip_memcpy_h2d(ctypes.c_void_p(p), raw.ctypes.data, raw.nbytes) == 0
+            return p + shift * es, val, cols + pad, rows * (cols + pad)
+
+        ta, tb = layout[0] == "t", layout[1] == "t"
+        pa, va, lda, sa = operand(*((K, M) if ta else (M, K)), batch)
+        pb, vb, ldb, sb = operand(*((N, K) if tb else (K, N)), 1 if share_b else batch)
+        self.A = va.transpose(0, 2, 1) if ta else va
+        self.B = vb.transpose(0, 2, 1) if tb else vb
+        d = self.d = Desc(dtype=dtype, M=M, N=N, K=K, a=pa, b=pb)
+        d.a_stride_m, d.a_stride_k = (1, lda) if ta else (lda, 1)
+        d.b_stride_k, d.b_stride_n = (1, ldb) if tb else (ldb, 1)
+        if batch > 1:
+            d.batch_ndim, d.batch_shape[0], d.a_batch_stride[0], d.b_batch_stride[0] = 1, batch, sa, 0 if share_b else sb
+        self.exact = self.A @ self.B
+        self.bound = (K + 2) * EPS32 * (np.abs(self.A) @ np.abs(self.B)) + 1e-30
+        self.n = batch * M * N
+        d.c = self.c = self.put(np.full(self.n + 4, 7.0, np.float32))
+
+    def put(self, x):
+        p = self.dev.alloc(x.nbytes)
+        assert self.lib.ormi_hip_memcpy_h2d(ctypes.c_void_p(p), x.ctypes.data, x.nbytes) == 0
+        return p
+
+    def get(self, p=None):
+        raw = self.dev.get(p or self.c, (self.n + 4) * 4).view(np.float32)
+        if p is None:
+            assert np.all(raw[self.n:] == 7.0)  # nothing past the output
+        return raw[:self.n].reshape(self.batch, self.M, self.N)
+
+    def run(self, epi=None):
+        rc = self.lib.ormi_hip_gemm_ex(ctypes.byref(self.d), ctypes.byref(epi) if epi else None)
+        assert rc == 0, self.lib.ormi_hip_last_error()
+
+    def check(self, got, want=None, extra=0.0):
+        want = self.exact if want is None else want
+        assert np.all(np.abs(got - want) <= self.bound * (1 + extra) + extra * EPS32 * (1 + np.abs(want)))
+
+
+@pytest.fixture
+def product(cabi):
+    made = []
+
+    def make(*a, **k):
+        made.append(Product(cabi, *a, **k))
+        return made[-1]
+
+    yield make
+    for p in made:
+        p.dev.free()
+
+
+SIZES = [(1, 4, 1), (1, 1, 5), (3, 3, 40), (1, 5, 31), (4, 1, 33), (15, 64, 32), (16, 65, 33), (17, 63, 95), (16, 4097, 160), (12, 1000, 2049),
+         (33, 31, 127), (65, 17, 300), (61, 1690, 49), (64, 64, 4096), (100, 130, 70), (200, 1003, 205), (500, 16, 513), (1001, 1003, 45)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
+@pytest.mark.parametrize("dtype", [F32, BF16, F16])
+def test_sizes(hip, product, dtype, layout):
+    for M, N, K in SIZES:
+        p = product(dtype, layout, M, N, K)
+        p.run()
+        p.check(p.get())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pad,shift", [(0, 1), (1, 0), (3, 3)])
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
+@pytest.mark.parametrize("dtype", [F32, BF16, F16])
+def test_unaligned_operands(hip, product, dtype, layout, pad, shift):
+    for M, N, K in [(16, 64, 64), (40, 96, 128), (256, 128, 96), (2, 4, 65)]:
+        p = product(dtype, layout, M, N, K, pad=pad, shift=shift)
+        p.run()
+        p.check(p.get())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("share_b", [False, True])
+@pytest.mark.parametrize("dtype,layout", [(F16, "nt"), (F32, "nn"), (BF16, "tn")])
+def test_batches(hip, product, dtype, layout, share_b):
+    for b, M, N, K in [(3, 50, 33, 65), (48, 19, 70, 30), (2, 16, 700, 1000)]:
+        p = product(dtype, layout, M, N, K, batch=b, share_b=share_b)
+        p.run()
+        p.check(p.get())
+
+
+@pytest.mark.gpu
+def test_non_finite_values_stay_in_their_rows(hip, product, cabi):
+    """inf and NaN past a row's or the k-range's end reach no other element: the
+    last partial k-step and the clamped rows must not multiply them in."""
+    for dtype, layout in [(F32, "nn"), (BF16, "nn"), (F16, "tn"), (F32, "nt")]:
+        M, N, K = 18, 70, 37
+        p = product(dtype, layout, M, N, K, pad=5)
+        ta, tb = layout[0] == "t", layout[1] == "t"
+        es = 4 if dtype == F32 else 2
+        nan = {F32: np.uint32(0x7FC00000), BF16: np.uint16(0x7FC0), F16: np.uint16(0x7E00)}[dtype]
+        pads = np.full(5, nan)
+        for base, rows, ld, cols in ((p.d.a, K if ta else M, (M if ta else K) + 5, M if ta else K),
+                                     (p.d.b, N if tb else K, (K if tb else N) + 5, K if tb else N)):
+            for r in range(rows):
+                assert cabi.ormi_hip_memcpy_h2d(ctypes.c_void_p(base + (r * ld + cols) * es), pads.ctypes.data, pads.nbytes) == 0
+        p.run()
+        p.check(p.get())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(12, 1000, 2049), (33, 31, 127), (61, 1690, 49), (300, 70, 500)])
+@pytest.mark.parametrize("dtype", [F32, BF16])
+def test_epilogues(hip, product, dtype, M, N, K):
+    rng = np.random.default_rng(3)
+    D = rng.standard_normal((M, N)).astype(np.float32)
+    s = np.float32(-0.37)
+    p = product(dtype, "nn", M, N, K)
+    d, ps = p.put(np.concatenate([D.reshape(-1), np.zeros(4, np.float32)])), p.put(np.array([s], np.float32))
+    v = p.exact[0]
+    for form, want in ((0, D + v * s), (1, D - v * s), (2, v * s - D)):
+        p.run(Epi(kind=1, form=form, s=ps, d=d, d_stride_m=N, d_stride_n=1))
+        p.check(p.get()[0], want, 4.0)
+    aux = p.put(np.full(p.n + 4, 7.0, np.float32))
+    p.run(Epi(kind=2, fn=1, aux=aux))
+    p.check(p.get()[0], np.maximum(v, 0))
+    p.check(p.get(aux)[0], v)
+    p.run(Epi(kind=3, fn=0, d=d, d_stride_m=N, d_stride_n=1))
+    assert np.all(np.abs(p.get()[0] - v * D) <= (p.bound[0] + EPS32 * np.abs(v)) * np.abs(D) * 1.01 + 1e-30)
+    # In place: each element's D is read before its product is stored there.
+    p2 = product(dtype, "nn", M, N, K)
+    start = np.concatenate([D.reshape(-1), np.full(4, 7.0, np.float32)])
+    assert p2.lib.ormi_hip_memcpy_h2d(ctypes.c_void_p(p2.c), start.ctypes.data, start.nbytes) == 0
+    p2.run(Epi(kind=1, form=1, s=ps, d=p2.c, d_stride_m=N, d_stride_n=1))
+    p2.check(p2.get()[0], D - p2.exact[0] * s, 4.0)

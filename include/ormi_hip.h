@@ -216,6 +216,13 @@ typedef struct ormi_gemm_epilogue {
 } ormi_gemm_epilogue;
 int ormi_hip_gemm_ex(const ormi_gemm_desc* desc, const ormi_gemm_epilogue* epi);
 
+/* ormi_hip_gemm_ex of a bf16 or f16 product with a UNARY epilogue that also
+ * stores fn(v), rounded to nearest even to cast_dtype (ORMI_DTYPE_BF16 or
+ * ORMI_DTYPE_F16), to cast, laid out like C: the activation a next 16-bit
+ * layer reads, without a conversion pass over C. cast must not overlap C, aux
+ * or an operand. */
+int ormi_hip_gemm_ex_cast(const ormi_gemm_desc* desc, const ormi_gemm_epilogue* epi, void* cast, int cast_dtype);
+
 /* ormi_hip_gemm_ex without any device allocation. No counterpart in the
  * reference: it is for callers that cannot allocate device memory (tight
  * serving loops, harnesses that forbid hipMalloc). Same kernels, same results

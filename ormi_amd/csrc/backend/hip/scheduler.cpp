@@ -466,6 +466,27 @@ namespace ormi::hip {
         return true;
     }
 
+    // A cast to 16 bits of an activation of a 16-bit product, f(p) rounded: the
+    // activation's GEMM stores the rounded values too (ormi_hip_gemm_ex_cast),
+    // besides p and f(p), which a later reader may want as before.
+    static bool match_cast(const NodePtr& n, EpilogueMatch& m) {
+        if (n->op != OpEnum::CAST || n->is_realized() || (n->dtype != DType::BFloat16 && n->dtype != DType::Float16)) return false;
+        if (!match_epilogue(n->parents[0], m) || m.kind != ORMI_GEMM_EPI_UNARY) return false;
+        const DType a = m.g->parents[0]->dtype, b = m.g->parents[1]->dtype;
+        return a == b && (a == DType::BFloat16 || a == DType::Float16);
+    }
+    static bool run_gemm_cast(const NodePtr& n, const EpilogueMatch& m) {
+        PreparedGemm pg;
+        if (!prepare_epilogue(n->parents[0], m, pg)) return false;
+        auto out = empty(n->view.shape, DeviceEnum::HIP, n->dtype);
+        if (!pg.empty)
+            ORMI_HIP_CHECK(ormi_hip_gemm_ex_cast(&pg.d, &pg.e, out->ptr, n->dtype == DType::BFloat16 ? ORMI_DTYPE_BF16 : ORMI_DTYPE_F16));
+        commit(pg);
+        n->data = out;
+        n->view.strides = calc_contiguous_strides(n->view.shape);
+        return true;
+    }
+
     // Forward activations of GEMM products, indexed once per top-level
     // realize. Autograd can reach a product p first through f'(p), as the D of
     // a backward epilogue, when a weight update is realized before the loss;
@@ -642,6 +663,7 @@ namespace ormi::hip {
         {
             EpilogueMatch m;
             if (match_epilogue(root, m) && run_gemm_epilogue(root, m)) return;
+            if (match_cast(root, m) && run_gemm_cast(root, m)) return;
         }
         if (const NodePtr r = epilogue_reduction(root)) {
             reduce_handler(r, r->op == OpEnum::SUM ? ReduceOp::Sum : ReduceOp::Max, root);
@@ -671,7 +693,7 @@ namespace ormi::hip {
         if (is_view_op(n->op)) return {n->parents[0]};
         if (fusible_root(*n)) {
             EpilogueMatch m;
-            if (match_epilogue(n, m)) {
+            if (match_epilogue(n, m) || match_cast(n, m)) {
                 std::vector<NodePtr> deps{m.g->parents[0], m.g->parents[1]};
                 if (m.d) deps.push_back(m.d);
                 if (m.s) deps.push_back(m.s);
@@ -703,7 +725,7 @@ namespace ormi::hip {
         }
         if (fusible_root(*n)) {
             EpilogueMatch m;
-            if (!match_epilogue(n, m) && !epilogue_reduction(n) && reads_a_reduction(region_frontier(n)) && run_row_program(n)) return;
+            if (!match_epilogue(n, m) && !match_cast(n, m) && !epilogue_reduction(n) && reads_a_reduction(region_frontier(n)) && run_row_program(n)) return;
             run_map(n);
             return;
         }
@@ -761,7 +783,7 @@ namespace ormi::hip {
             std::vector<NodePtr> open;
             for (const auto& r : roots) {
                 EpilogueMatch m;
-                if (r && !r->is_realized() && !match_epilogue(r, m)) open.push_back(r);
+                if (r && !r->is_realized() && !match_epilogue(r, m) && !match_cast(r, m)) open.push_back(r);
             }
             if (open.size() >= 2) realize_row_groups(open);
         }
@@ -774,7 +796,7 @@ namespace ormi::hip {
             if (!r || r->is_realized() || !seen.insert(r.get()).second) continue;
             if (r->device.type != DeviceEnum::HIP) throw std::runtime_error("HIP scheduler: node belongs to another device.");
             EpilogueMatch m;
-            if (!fusible_interior(*r) || match_epilogue(r, m) || epilogue_reduction(r)) {
+            if (!fusible_interior(*r) || match_epilogue(r, m) || match_cast(r, m) || epilogue_reduction(r)) {
                 rest.push_back(r);
                 continue;
             }

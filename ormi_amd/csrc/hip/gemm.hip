@@ -338,7 +338,13 @@ struct FinishParams {
     Epi epi;
 };
 
-template <bool VEC>
+// One partial at a time, a thread of a split product waits out a memory latency
+// per split: the finish of 12 x 4096 with 4 splits took 4.8 us.
+constexpr int kFinishSplits = 4;
+
+// W: columns per thread. Small outputs take one, so that an activation's
+// arithmetic is spread over more waves instead of repeated in each.
+template <bool VEC, int W>
 __global__ __launch_bounds__(256) void gemm_finish_kernel(FinishParams f) {
     const Epi& e = f.epi;
     const float sv = e.s ? *e.s : 0.0f;
@@ -355,33 +361,48 @@ __global__ __launch_bounds__(256) void gemm_finish_kernel(FinishParams f) {
             d_off += (long long)m * e.d_sm;
         }
         const long long base = (long long)row * f.N;
-        for (int col0 = (blockIdx.x * blockDim.x + threadIdx.x) * 4; col0 < f.N; col0 += gridDim.x * blockDim.x * 4) {
-            const int cnt = min(4, f.N - col0);
-            float v[4] = {0.0f, 0.0f, 0.0f, 0.0f}, dv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int col0 = (blockIdx.x * blockDim.x + threadIdx.x) * W; col0 < f.N; col0 += gridDim.x * blockDim.x * W) {
+            const int cnt = min(W, f.N - col0);
+            float v[W], dv[W];
+#pragma unroll
+            for (int k = 0; k < W; ++k) v[k] = dv[k] = 0.0f;
             if (reads_d) {
 #pragma unroll
-                for (int k = 0; k < 4; ++k)
+                for (int k = 0; k < W; ++k)
                     if (k < cnt) dv[k] = e.d[d_off + (long long)(col0 + k) * e.d_sn];
             }
-            for (int q = 0; q < f.splits; ++q) {
-                const float* w = f.ws + (long long)q * f.n + base + col0;
-                float t[4];
-                if (VEC) {
-                    const ormi_f4 x = *(const ormi_f4*)w;
+            // Partials of kFinishSplits splits in flight, added in split order.
+            for (int q0 = 0; q0 < f.splits; q0 += kFinishSplits) {
+                float t[kFinishSplits][W];
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) t[k] = x[k];
-                } else {
+                for (int j = 0; j < kFinishSplits; ++j) {
+                    if (q0 + j >= f.splits) continue;
+                    const float* w = f.ws + (long long)(q0 + j) * f.n + base + col0;
+                    if constexpr (VEC) {
+                        const ormi_f4 x = *(const ormi_f4*)w;
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) t[k] = k < cnt ? w[k] : 0.0f;
+                        for (int k = 0; k < W; ++k) t[j][k] = x[k];
+                    } else {
+#pragma unroll
+                        for (int k = 0; k < W; ++k) t[j][k] = k < cnt ? w[k] : 0.0f;
+                    }
                 }
 #pragma unroll
-                for (int k = 0; k < 4; ++k) v[k] = q == 0 ? t[k] : v[k] + t[k];
-            }
-            if (VEC && e.kind == ORMI_GEMM_EPI_NONE) {
-                *(ormi_f4*)(f.c + base + col0) = ormi_f4{v[0], v[1], v[2], v[3]};
-            } else {
+                for (int j = 0; j < kFinishSplits; ++j) {
+                    if (q0 + j >= f.splits) continue;
 #pragma unroll
-                for (int k = 0; k < 4; ++k)
+                    for (int k = 0; k < W; ++k) v[k] = q0 + j == 0 ? t[j][k] : v[k] + t[j][k];
+                }
+            }
+            if constexpr (VEC) {
+                if (e.kind == ORMI_GEMM_EPI_NONE) {
+                    *(ormi_f4*)(f.c + base + col0) = ormi_f4{v[0], v[1], v[2], v[3]};
+                    continue;
+                }
+            }
+            {
+#pragma unroll
+                for (int k = 0; k < W; ++k)
                     if (k < cnt) epi_store(e, sv, f.c, e.aux, base + col0 + k, dv[k], v[k]);
             }
         }
@@ -390,9 +411,9 @@ __global__ __launch_bounds__(256) void gemm_finish_kernel(FinishParams f) {
 
 // The finish pass without an epilogue, for C contiguous over the n elements
 // of a split and 16-byte aligned (n % 4 == 0): a flat grid-stride walk over
-// float4 groups, U groups per thread with every split's loads issued before
-// the sums, in split order like gemm_finish_kernel.
-template <int U>
+// float4 groups, U groups of Q splits per thread in flight, summed in split
+// order like gemm_finish_kernel.
+template <int U, int Q>
 __global__ __launch_bounds__(256) void gemm_finish_flat_kernel(float* __restrict__ c, const float* __restrict__ ws,
                                                                long long n4, int splits) {
     const long long stride = (long long)gridDim.x * blockDim.x;
@@ -405,15 +426,21 @@ __global__ __launch_bounds__(256) void gemm_finish_flat_kernel(float* __restrict
             const long long g = g0 + u * stride;
             if (g < n4) v[u] = w[g];
         }
-        for (int q = 1; q < splits; ++q) {
-            ormi_f4 t[U];
+        for (int q0 = 1; q0 < splits; q0 += Q) {
+            ormi_f4 t[Q][U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const long long g = g0 + u * stride;
-                if (g < n4) t[u] = w[q * n4 + g];
+            for (int j = 0; j < Q; ++j)
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const long long g = g0 + u * stride;
+                    if (q0 + j < splits && g < n4) t[j][u] = w[(q0 + j) * n4 + g];
+                }
+#pragma unroll
+            for (int j = 0; j < Q; ++j) {
+                if (q0 + j >= splits) continue;
+#pragma unroll
+                for (int u = 0; u < U; ++u) v[u] += t[j][u];
             }
-#pragma unroll
-            for (int u = 0; u < U; ++u) v[u] += t[u];
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -1421,16 +1448,22 @@ static void launch_finish(const ormi_gemm_desc* d, const float* ws, int splits, 
     f.epi = epi;
     const bool vec = d->N % 4 == 0 && ((uintptr_t)d->c & 15u) == 0 && ((uintptr_t)epi.aux & 15u) == 0;
     if (vec && epi.kind == ORMI_GEMM_EPI_NONE) {
-        constexpr int U = 4;
+        // Few groups: one per thread, so that every thread has some, and more
+        // splits of it in flight.
         const long long n4 = f.n / 4;
-        const long long blocks = std::max(1LL, std::min((n4 + 256LL * U - 1) / (256LL * U), (long long)compute_units() * 8));
-        gemm_finish_flat_kernel<U><<<(unsigned)blocks, 256>>>(f.c, ws, n4, splits);
+        auto blocks = [&](int u) {
+            return (unsigned)std::max(1LL, std::min((n4 + 256LL * u - 1) / (256LL * u), (long long)compute_units() * 8));
+        };
+        if (n4 < 256LL * 4 * compute_units()) gemm_finish_flat_kernel<1, 8><<<blocks(1), 256>>>(f.c, ws, n4, splits);
+        else gemm_finish_flat_kernel<4, 1><<<blocks(4), 256>>>(f.c, ws, n4, splits);
         return;
     }
-    const int gx = std::min((d->N + 1023) / 1024, 64);
+    const bool small = f.n < 256LL * 4 * 4 * compute_units() && epi.kind != ORMI_GEMM_EPI_NONE;
+    const int gx = small ? std::min((d->N + 255) / 256, 64) : std::min((d->N + 1023) / 1024, 64);
     const int gy = std::max(1, std::min({f.rows, compute_units() * 32 / gx, 65535}));
-    if (vec) gemm_finish_kernel<true><<<dim3(gx, gy), 256>>>(f);
-    else gemm_finish_kernel<false><<<dim3(gx, gy), 256>>>(f);
+    if (small) gemm_finish_kernel<false, 1><<<dim3(gx, gy), 256>>>(f);
+    else if (vec) gemm_finish_kernel<true, 4><<<dim3(gx, gy), 256>>>(f);
+    else gemm_finish_kernel<false, 4><<<dim3(gx, gy), 256>>>(f);
 }
 }  // namespace ormi_hip
 
@@ -1469,12 +1502,15 @@ static int gemm_check(const ormi_gemm_desc* d, const ormi_gemm_epilogue* epi_in,
     return make_epi(d, epi_in, batch, epi);
 }
 
-static int gemm_run(const ormi_gemm_desc* d, const ormi_gemm_epilogue* epi_in, bool noalloc) {
+static int gemm_run(const ormi_gemm_desc* d, const ormi_gemm_epilogue* epi_in, bool noalloc, unsigned short* cast = nullptr,
+                    int cast_dtype = 0) {
     long long batch = 1;
     Epi epi;
     bool nothing = false;
     int rc = gemm_check(d, epi_in, &batch, &epi, &nothing);
     if (rc != ORMI_HIP_OK || nothing) return rc;
+    epi.cast = cast;
+    epi.cast_dtype = cast_dtype;
     rc = ensure_init();
     if (rc != ORMI_HIP_OK) return rc;
     rc = drain_queue();
@@ -1952,6 +1988,14 @@ static int gemm_run_locked(const ormi_gemm_desc* d, const Epi& epi, long long ba
 }  // namespace ormi_hip
 
 extern "C" int ormi_hip_gemm(const ormi_gemm_desc* d) { return gemm_run(d, nullptr, false); }
+
+extern "C" int ormi_hip_gemm_ex_cast(const ormi_gemm_desc* d, const ormi_gemm_epilogue* epi, void* cast, int cast_dtype) {
+    if (!d || (d->dtype != ORMI_DTYPE_BF16 && d->dtype != ORMI_DTYPE_F16) || !epi || epi->kind != ORMI_GEMM_EPI_UNARY)
+        return fail(ORMI_HIP_ERR_INVALID, "ormi_hip_gemm_ex_cast: a 16-bit product with a UNARY epilogue is needed");
+    if ((cast_dtype != ORMI_DTYPE_BF16 && cast_dtype != ORMI_DTYPE_F16) || !cast || ((uintptr_t)cast & 1u) != 0)
+        return fail(ORMI_HIP_ERR_INVALID, "ormi_hip_gemm_ex_cast: the converted output must be aligned bf16 or f16 memory");
+    return gemm_run(d, epi, false, (unsigned short*)cast, cast_dtype);
+}
 
 extern "C" int ormi_hip_gemm_ex(const ormi_gemm_desc* d, const ormi_gemm_epilogue* epi) { return gemm_run(d, epi, false); }
 

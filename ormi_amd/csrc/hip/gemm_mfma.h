@@ -44,6 +44,8 @@ struct Epi {
     long long d_sm, d_sn;
     long long d_bs[ORMI_GEMM_MAX_BATCH_DIMS];
     float* aux;
+    unsigned short* cast;  // UNARY: also store fn(v) as cast_dtype (bf16 or f16), or null
+    int cast_dtype;
 };
 
 struct GemmParams {
@@ -146,7 +148,9 @@ __device__ __forceinline__ void epi_store(const Epi& e, float sv, float* c, floa
         }
         case ORMI_GEMM_EPI_UNARY:
             if (aux) aux[ci] = v;
-            c[ci] = epi_fn(e.fn, v);
+            v = epi_fn(e.fn, v);
+            c[ci] = v;
+            if (e.cast) e.cast[ci] = e.cast_dtype == ORMI_DTYPE_BF16 ? ormi_f32_to_bf16(v) : ormi_f32_to_f16(v);
             break;
         case ORMI_GEMM_EPI_MUL_FN_D:
             c[ci] = v * epi_fn(e.fn, dv);

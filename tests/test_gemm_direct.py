@@ -184,3 +184,40 @@ def test_epilogues(hip, product, dtype, M, N, K):
     assert p2.lib.ormi_hip_memcpy_h2d(ctypes.c_void_p(p2.c), start.ctypes.data, start.nbytes) == 0
     p2.run(Epi(kind=1, form=1, s=ps, d=p2.c, d_stride_m=N, d_stride_n=1))
     p2.check(p2.get()[0], D - p2.exact[0] * s, 4.0)
+
+
+# ------------------------------------------------- activation and its cast --
+def test_cast_entry_checks_its_arguments(cabi):
+    d, e = Desc(dtype=BF16, M=4, N=4, K=4, a=256, a_stride_m=4, a_stride_k=1, b=512, b_stride_k=4, b_stride_n=1, c=1024), Epi(kind=2, fn=7)
+
+    def call(desc=d, epi=e, cast=2048, dtype=BF16):
+        return cabi.ormi_hip_gemm_ex_cast(ctypes.byref(desc), ctypes.byref(epi) if epi else None, ctypes.c_void_p(cast), dtype)
+
+    f32 = Desc.from_buffer_copy(d)
+    f32.dtype = F32
+    assert call(desc=f32) == 3 and call(epi=None) == 3 and call(epi=Epi(kind=1, d=256)) == 3
+    assert call(cast=None) == 3 and call(cast=2049) == 3 and call(dtype=F32) == 3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fn", ["gelu", "relu", "tanh", "sigmoid"])
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("M,K,N", [(12, 512, 1000), (5, 333, 77), (256, 1024, 512), (300, 2048, 2048), (3, 40, 7)])
+def test_activation_and_its_cast_from_one_product(ob, hip, M, K, N, dtype, fn):
+    """The rounded activation comes from the GEMM, with the bits of the separate
+    cast, and the product and the activation hold their buffers as well."""
+    from ormi_amd import Tensor
+
+    rng = np.random.default_rng(M + N)
+    x = Tensor(rng.standard_normal((M, K)).astype(np.float32), hip, dtype=dtype)
+    w = Tensor((rng.standard_normal((K, N)) / 16).astype(np.float32), hip, dtype=dtype)
+    p = x @ w
+    act = getattr(p, fn)()
+    h = act.astype(dtype)
+    before = ob._kernel_launches()
+    h.realize()
+    assert ob._kernel_launches() == before and p._node.is_realized and act._node.is_realized
+    q = (x @ w).realize()
+    act2 = getattr(q, fn)().realize()
+    assert np.array_equal(p.numpy(), q.numpy()) and np.array_equal(act.numpy(), act2.numpy())
+    assert np.array_equal(h.numpy(), act2.astype(dtype).numpy())

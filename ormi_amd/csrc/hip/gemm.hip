@@ -1740,7 +1740,8 @@ static int gemm_packed_locked(const ormi_gemm_desc* d, const Epi& epi, long long
 //     quarter) of the compute units, up to 2^31 multiply-adds (1024^3 bf16
 //     17.6 -> 12.0 us, 512^3 8.8 -> 5.4, 12 x 8192 x 2048 15.1 -> 12.3; past the
 //     line 2048^3 26 against 59, 200 x 4096^2 22 against 44, fp32 1024^3 26.6
-//     against 25.7);
+//     against 25.7), except where K is long enough to feed the tiles' splits
+//     (40 x 4096^2 16.1 against 18.2, 64 x 1024 x 8192 13.0 against 14.1);
 //   * otherwise packing, the register-staged kernels or the generic one would
 //     run: up to 2.7e9 multiply-adds in 16 bits (1001 x 1003 x 1005 34.4 -> 20.2,
 //     6 x 1544 x 2648 25.8 -> 12.4, 1500^3 47 against 70 us) and 2^33 in fp32
@@ -1755,7 +1756,9 @@ static bool takes_direct(const ormi_gemm_desc* d, long long batch, bool fast) {
     const long long macs = batch * d->M * d->N * (long long)d->K;
     const long long t128 = batch * ((d->M + 127) / 128) * ((d->N + 127) / 128);
     const bool f32 = d->dtype == ORMI_DTYPE_F32;
-    if (fast && d->K % (f32 ? 32 : 64) == 0) return t128 < (f32 ? compute_units() / 4 : compute_units() / 3) && macs <= (1LL << 31);
+    if (fast && d->K % (f32 ? 32 : 64) == 0)
+        return t128 < (f32 ? compute_units() / 4 : compute_units() / 3) && macs <= (1LL << 31) &&
+               (d->K < 4096 || d->M <= 16 || d->N <= 16);
     return macs <= (f32 ? 1LL << 33 : 5LL << 29);
 }
 

@@ -341,7 +341,8 @@ void launch(const GemmParams& p, dim3 grid, int waves, bool a_kc, bool b_kc) {
 }
 template <typename Tr>
 void launch_cfg(int mt, int nt, const GemmParams& p, dim3 grid, int waves, bool a_kc, bool b_kc) {
-    if (mt == 1) launch<Tr, 1, 4>(p, grid, waves, a_kc, b_kc);
+    if (mt == 1 && nt == 2) launch<Tr, 1, 2>(p, grid, waves, a_kc, b_kc);
+    else if (mt == 1) launch<Tr, 1, 4>(p, grid, waves, a_kc, b_kc);
     else if (nt == 1) launch<Tr, 4, 1>(p, grid, waves, a_kc, b_kc);
     else if (mt == 2 && nt == 2) launch<Tr, 2, 2>(p, grid, waves, a_kc, b_kc);
     else if (mt == 2) launch<Tr, 2, 4>(p, grid, waves, a_kc, b_kc);
@@ -359,7 +360,12 @@ DirectPlan gemm_direct_plan(const ormi_gemm_desc* d, long long batch, bool a_kc,
     auto tiles = [&](int mt, int nt) {
         return (long long)((d->M + 16 * mt - 1) / (16 * mt)) * ((d->N + 16 * nt - 1) / (16 * nt)) * batch;
     };
-    if (d->M <= 16) r.mt = 1, r.nt = 4;
+    // Up to 16 rows: 64 columns per work-group, a whole cache line of each k-row of
+    // 16-bit weights; 32 where the weights are few, for twice the work-groups
+    // (bf16 12 x 1000 x 4096 9.4 -> 8.3 us, 6 x 1544 x 2648 12.4 -> 10.3, fp32
+    // 16 x 3689 x 640 9.0 -> 6.9; 16 x 5096 x 2656 13.3 -> 13.7, 12 x 4096 x 8192
+    // 19.5 -> 24).
+    if (d->M <= 16) r.mt = 1, r.nt = (long long)d->N * d->K < (3LL << 22) ? 2 : 4;
     else if (d->N <= 16) r.mt = 4, r.nt = 1;
     else if (tiles(4, 4) >= (f32 ? cus : 2 * cus)) r.mt = 4, r.nt = 4;
     else if (tiles(2, 4) >= 3 * cus / 8) r.mt = 2, r.nt = 4;
@@ -381,7 +387,7 @@ DirectPlan gemm_direct_plan(const ormi_gemm_desc* d, long long batch, bool a_kc,
     const long long enough = f32 && r.mt * r.nt == 16 ? 1LL << 40 : 6 * cus;
     while (r.waves < most && t * r.waves < enough && steps >= 4LL * r.waves) r.waves *= 2;
     const long long deep = t < 3 * cus / 8 || r.mt == 1 || r.nt == 1 ? 4 : f32 ? 16 : 8;
-    while (r.splits < 8 && t * r.splits < 3 * cus / 4 && steps >= deep * r.waves * r.splits) r.splits *= 2;
+    while (r.splits < 8 && t * r.splits < (r.mt == 1 && r.nt == 2 && !f32 ? cus / 2 : 3 * cus / 4) && steps >= deep * r.waves * r.splits) r.splits *= 2;
     if (batch * r.splits > 65535) r.splits = 1;
     return r;
 }

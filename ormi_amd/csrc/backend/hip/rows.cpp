@@ -21,7 +21,6 @@
 // every per-row value that a full node reads, so that what reads them later
 // finds buffers.
 #include <algorithm>
-#include <unordered_map>
 #include <vector>
 
 #include "backend/hip/hip_backend.h"
@@ -93,6 +92,7 @@ namespace ormi::hip {
                 keep_ = s.s;
                 for (int d = nd - s.k; d < nd; ++d) keep_[d] = 1;
                 kept_.assign(s.s.begin(), s.s.end() - s.k);
+                items.reserve(32);
             }
 
             // Adds root (a node of the program's space); false, with the
@@ -132,13 +132,27 @@ namespace ormi::hip {
 
         private:
             std::vector<int> keep_, kept_;
-            std::unordered_map<const Node*, int> index_[2];  // by context: right-aligned to S, or to the kept shape
+            // Items by node, per context (right-aligned to S, or to the kept
+            // shape): at most kMaxItems and their views, searched linearly.
+            struct Index {
+                SmallVec<std::pair<const Node*, int>, 64> at;
+                int find(const Node* n) const {
+                    for (size_t i = 0; i < at.size(); ++i)
+                        if (at[i].first == n) return at[i].second;
+                    return -1;
+                }
+                void add(const Node* n, int id) { at.push_back({n, id}); }
+                void clear() {
+                    while (!at.empty()) at.pop_back();
+                }
+            };
+            Index index_[2];
             bool plan_only_, over_ = false, touched_ = false;
 
             void reindex() {
                 index_[0].clear();
                 index_[1].clear();
-                for (size_t i = 0; i < items.size(); ++i) index_[ctx(items[i])].emplace(items[i].n.get(), (int)i);
+                for (size_t i = 0; i < items.size(); ++i) index_[ctx(items[i])].add(items[i].n.get(), (int)i);
             }
             static int ctx(const Item& x) { return x.leaf ? (x.kept_ctx ? 1 : 0) : x.form == Kept ? 1 : 0; }
             // The form of a shape read right-aligned to S (or, in_kept, to the
@@ -175,7 +189,7 @@ namespace ormi::hip {
                 }
                 items.push_back(std::move(x));
                 const int id = (int)items.size() - 1;
-                index_[ctx(items[id])].emplace(items[id].n.get(), id);
+                index_[ctx(items[id])].add(items[id].n.get(), id);
                 return id;
             }
             // A leaf varies along the row unless it broadcasts over the last k dims.
@@ -209,9 +223,9 @@ namespace ormi::hip {
             // a node may also turn out to be Scalar). -1 past the limits.
             int visit(const NodePtr& n, Form f) {
                 const bool in_kept = f == Kept;
-                if (const auto it = index_[in_kept].find(n.get()); it != index_[in_kept].end()) {
-                    if (items[it->second].form != Scalar) touched_ = true;
-                    return it->second;
+                if (const int id = index_[in_kept].find(n.get()); id >= 0) {
+                    if (items[id].form != Scalar) touched_ = true;
+                    return id;
                 }
                 if (over_) return -1;
                 if (n->is_realized()) return leaf(n, in_kept);
@@ -254,20 +268,20 @@ namespace ormi::hip {
                 return leaf(n, in_kept);
             }
             int leaf_once(const NodePtr& p, bool in_kept) {
-                if (const auto it = index_[in_kept].find(p.get()); it != index_[in_kept].end()) {
-                    if (items[it->second].form != Scalar) touched_ = true;
-                    return it->second;
+                if (const int id = index_[in_kept].find(p.get()); id >= 0) {
+                    if (items[id].form != Scalar) touched_ = true;
+                    return id;
                 }
                 return leaf(p, in_kept);
             }
             int push_scalar(Item x) {
                 const int id = push(std::move(x));
-                if (id >= 0) index_[1].emplace(items[id].n.get(), id);
+                if (id >= 0) index_[1].add(items[id].n.get(), id);
                 return id;
             }
             // Node n (a view) is the value `id` renamed.
             int alias(const NodePtr& n, bool in_kept, int id) {
-                if (id >= 0) index_[in_kept].emplace(n.get(), id);
+                if (id >= 0) index_[in_kept].add(n.get(), id);
                 return id;
             }
         };
@@ -465,7 +479,10 @@ namespace ormi::hip {
                     else left.push_back(r);
                 *list = std::move(left);
             }
-            if (mine.size() >= 2 && b.worthwhile()) realize_rows(mine, sp);
+            if (mine.size() >= 2 && b.worthwhile()) {
+                if (b.frontier.empty()) run(b);
+                else realize_rows(mine, sp);
+            }
             rest = std::move(after);  // what came before the seed has no space of its own
         }
     }

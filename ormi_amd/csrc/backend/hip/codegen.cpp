@@ -1,5 +1,6 @@
-// hipRTC code generator for gfx950: fused element-wise maps, and row / column
-// reductions with a fused element-wise prologue.
+// hipRTC code generator for gfx950: fused element-wise maps, row / column
+// reductions with a fused element-wise prologue, and row programs (several
+// reductions over the rows of one shape and the values around them).
 //
 // Replaces the reference's NVRTC source builder (csrc/backend/cuda/compiler.cu:53-112)
 // and its atomic sum kernel (csrc/backend/cuda/kernels/reduce/sum.cu:29-66). Unlike

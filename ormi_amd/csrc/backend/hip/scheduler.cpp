@@ -11,6 +11,8 @@
 //                    recomputed by any later kernel that reads them;
 //   * SUM/MAX/ARGMAX -> the producing pointwise region is fused into the
 //                    reduction as its prologue;
+//   * several reductions over the same rows, with the pointwise values
+//                    around them -> one row program (rows.cpp);
 //   * MATMUL      -> both operands realized, MFMA GEMM.
 // Reductions and MATMUL are registered as graph breakers for DeviceEnum::HIP
 // (the reference's plugin point, csrc/backend/graph_breakers.h:12-14).
@@ -657,6 +659,26 @@ namespace ormi::hip {
         return false;
     }
 
+    // A product with a backward pass's seed, 1 * x with x a dense buffer of the
+    // product's shape, is x bit for bit: it aliases x's buffer instead of copying it
+    // (the gradient of sum(c * w) with respect to c, before c's own backward
+    // products: 13.8 us for 2048 x 4096).
+    static bool alias_times_one(const NodePtr& root) {
+        if (root->op != OpEnum::MUL || root->dtype != DType::Float32) return false;
+        for (int k = 0; k < 2; ++k) {
+            const NodePtr &u = root->parents[k], &x = root->parents[1 - k];
+            if (!u->is_realized() || !u->data->one || !x->is_realized()) continue;
+            if (x->data->dtype != DType::Float32 || x->device.type != DeviceEnum::HIP || x->view.shape != root->view.shape ||
+                x->view.strides != calc_contiguous_strides(root->view.shape) ||
+                (long long)x->data->numel() != shape_numel(root->view.shape))
+                continue;
+            root->data = x->data;
+            root->view.strides = x->view.strides;
+            return true;
+        }
+        return false;
+    }
+
     // An element-wise region: a matched GEMM epilogue, a reduction's store
     // epilogue, else one fused kernel.
     static void run_map(const NodePtr& root) {
@@ -670,6 +692,7 @@ namespace ormi::hip {
             return;
         }
         for (const auto& f : region_frontier(root)) realize(f);
+        if (alias_times_one(root)) return;
         const Expr e = build_expr(root, root->view.shape);
         auto out = empty(root->view.shape, DeviceEnum::HIP, root->dtype);
         root->data = out;

@@ -74,7 +74,10 @@ namespace ormi {
         static auto* cache = new std::map<std::pair<int, std::vector<int>>, std::shared_ptr<Buffer>>();
         std::lock_guard<std::mutex> lock(mu);
         auto& b = (*cache)[{(int)dev, shape}];
-        if (!b) b = ones(shape, dev);
+        if (!b) {
+            b = ones(shape, dev);
+            b->one = true;
+        }
         return b;
     }
 

@@ -16,6 +16,7 @@ namespace ormi {
         std::vector<int> shape;
         Device device;
         DType dtype;
+        bool one = false;  // a shared read-only 1.0 (a backward pass's seed)
 
         Buffer(void* p, size_t b, std::vector<int> s, Device d, DType dt = DType::Float32);
         ~Buffer();

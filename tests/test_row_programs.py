@@ -190,3 +190,25 @@ def test_deep_chain_of_rows(hip):
         X = X - X.max(1, keepdims=True) * 0.5
         want = want - want.max(1, keepdims=True) * np.float32(0.5)
     assert np.array_equal(X.numpy(), want)
+
+
+@pytest.mark.gpu
+def test_a_seed_times_a_buffer_is_the_buffer(ob, hip):
+    """The gradient of sum(c * w) with respect to c is w: no kernel copies it, and
+    the two backward products read it as it is; a transposed or broadcast w is
+    still multiplied out."""
+    rng = np.random.default_rng(5)
+    a, b, w = (rng.standard_normal(s).astype(np.float32) for s in ((40, 24), (24, 56), (40, 56)))
+    for wt in (Tensor(w, hip), Tensor(np.ascontiguousarray(w.T), hip).transpose(), Tensor(w[:1], hip)):
+        A, B = Tensor(a, hip, requires_grad=True), Tensor(b, hip, requires_grad=True)
+        total = ((A @ B) * wt).sum()
+        total.backward()
+        before = ob._kernel_launches()
+        realize_all(A.grad, B.grad)
+        if wt.op == ob.OpEnum.LEAF and wt.shape == (40, 56):
+            assert ob._kernel_launches() == before
+        full = np.broadcast_to(w[:1], w.shape) if wt.shape == (1, 56) else w
+        for got, want, scale in ((A.grad, full.astype(np.float64) @ b.T, np.abs(full) @ np.abs(b).T),
+                                 (B.grad, a.T.astype(np.float64) @ full, np.abs(a).T @ np.abs(full))):
+            assert np.all(np.abs(got.numpy() - want) <= 60 * EPS32 * scale)
+        total.zero_grad_graph()

@@ -403,7 +403,7 @@ __global__ __launch_bounds__(256) void gemm_finish_kernel(FinishParams f) {
             {
 #pragma unroll
                 for (int k = 0; k < W; ++k)
-                    if (k < cnt) epi_store(e, sv, f.c, e.aux, base + col0 + k, dv[k], v[k]);
+                    if (k < cnt) epi_store(e, sv, f.c, e.aux, e.cast, base + col0 + k, dv[k], v[k]);
             }
         }
     }
@@ -539,7 +539,8 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(GemmParams p) {
     if (row < p.M && col < p.N) {
         const Epi& e = p.epi;
         const float dv = epi_reads_d(e) ? e.d[d_off + row * e.d_sm + col * e.d_sn] : 0.0f;
-        epi_store(e, e.s ? *e.s : 0.0f, p.c + c_off, e.aux ? e.aux + c_off : nullptr, (long long)row * p.N + col, dv, acc);
+        epi_store(e, e.s ? *e.s : 0.0f, p.c + c_off, e.aux ? e.aux + c_off : nullptr, e.cast ? e.cast + c_off : nullptr,
+                  (long long)row * p.N + col, dv, acc);
     }
 }
 

@@ -295,6 +295,7 @@ __global__ __launch_bounds__((64 * kMostWaves<MT, NT>)) void gemm_direct_kernel(
     const float sv = e.s ? *e.s : 0.0f;
     float* const c = p.c + c_off;
     float* const aux = e.aux ? e.aux + c_off : nullptr;
+    unsigned short* const cast = e.cast ? e.cast + c_off : nullptr;
     for (int unit = w; unit < 4 * MT; unit += W) {
         const int i = unit / 4, t = unit % 4;
         float v[NT];
@@ -325,7 +326,7 @@ __global__ __launch_bounds__((64 * kMostWaves<MT, NT>)) void gemm_direct_kernel(
                 if (!ob.owns(j, p.N)) continue;
                 const int n = ob.mn(j);
                 const float dv = epi_reads_d(e) ? e.d[d_off + orow.mn(i) * e.d_sm + n * e.d_sn] : 0.0f;
-                epi_store(e, sv, c, aux, at + n, dv, v[j]);
+                epi_store(e, sv, c, aux, cast, at + n, dv, v[j]);
             }
         }
     }

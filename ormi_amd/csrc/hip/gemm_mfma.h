@@ -134,12 +134,14 @@ __host__ __device__ __forceinline__ bool epi_reads_d(const Epi& e) {
     return e.kind == ORMI_GEMM_EPI_ADD || e.kind == ORMI_GEMM_EPI_MUL_FN_D;
 }
 
-// Store product v of one output element: C[ci] (and aux[ci]) in C's layout;
-// dv is that element's D value (read beforehand when epi_reads_d), sv the
+// Store product v of one output element: C[ci] (and aux[ci], cast[ci]) in C's
+// layout, with ci counted from where those three point (a batch's kernel
+// advances them together); dv is that element's D value (read beforehand when epi_reads_d), sv the
 // scale s[0] when the epilogue has one. Every HIP translation unit is
 // compiled with -ffp-contract=off, so each operation below rounds on its own,
 // as in the unfused element-wise kernel.
-__device__ __forceinline__ void epi_store(const Epi& e, float sv, float* c, float* aux, long long ci, float dv, float v) {
+__device__ __forceinline__ void epi_store(const Epi& e, float sv, float* c, float* aux, unsigned short* cast, long long ci, float dv,
+                                          float v) {
     switch (e.kind) {
         case ORMI_GEMM_EPI_ADD: {
             const float t = e.s ? v * sv : v;
@@ -150,7 +152,7 @@ __device__ __forceinline__ void epi_store(const Epi& e, float sv, float* c, floa
             if (aux) aux[ci] = v;
             v = epi_fn(e.fn, v);
             c[ci] = v;
-            if (e.cast) e.cast[ci] = e.cast_dtype == ORMI_DTYPE_BF16 ? ormi_f32_to_bf16(v) : ormi_f32_to_f16(v);
+            if (cast) cast[ci] = e.cast_dtype == ORMI_DTYPE_BF16 ? ormi_f32_to_bf16(v) : ormi_f32_to_f16(v);
             break;
         case ORMI_GEMM_EPI_MUL_FN_D:
             c[ci] = v * epi_fn(e.fn, dv);

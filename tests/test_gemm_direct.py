@@ -221,3 +221,32 @@ def test_activation_and_its_cast_from_one_product(ob, hip, M, K, N, dtype, fn):
     act2 = getattr(q, fn)().realize()
     assert np.array_equal(p.numpy(), q.numpy()) and np.array_equal(act.numpy(), act2.numpy())
     assert np.array_equal(h.numpy(), act2.astype(dtype).numpy())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cast_dtype", [BF16, F16])
+@pytest.mark.parametrize("dtype", [BF16, F16])
+@pytest.mark.parametrize("batch,M,N,K,layout,step", [
+    (3, 50, 33, 65, "nt", 1),      # direct, one pass
+    (2, 16, 700, 4096, "nn", 1),   # direct, split over K: the finish pass
+    (3, 17, 40, 31, "nn", 2),      # no unit stride, small: the generic kernel
+    (2, 200, 320, 300, "nn", 2),   # no unit stride, packed: the tiles and the finish pass
+    (2, 64, 256, 4096, "nt", 1),   # the tiles and the finish pass
+])
+def test_cast_of_a_batch_is_laid_out_like_c(hip, product, cabi, dtype, cast_dtype, batch, M, N, K, layout, step):
+    """Every matrix of the batch has its own rounded values, bit for bit those
+    of C, and nothing is written past the last."""
+    p = product(dtype, layout, M, N, K * step, batch=batch)
+    if step > 1:  # every step-th k of A
+        p.d.K, p.d.a_stride_k = K, step
+        a, b = p.A[:, :, ::step], p.B[:, :K]
+        p.exact, p.bound = a @ b, (K + 2) * EPS32 * (np.abs(a) @ np.abs(b)) + 1e-30
+    aux, out = p.put(np.full(p.n + 4, 7.0, np.float32)), p.put(np.full(p.n + 8, 0x1234, np.uint16))
+    e = Epi(kind=2, fn=1, aux=aux)
+    rc = cabi.ormi_hip_gemm_ex_cast(ctypes.byref(p.d), ctypes.byref(e), ctypes.c_void_p(out), cast_dtype)
+    assert rc == 0, cabi.ormi_hip_last_error()
+    c = p.get()
+    p.check(p.get(aux))
+    p.check(c, np.maximum(p.exact, 0))
+    got = p.dev.get(out, (p.n + 8) * 2).view(np.uint16)
+    assert np.array_equal(got[:p.n], storage(c.reshape(-1), cast_dtype)[0].view(np.uint16)) and np.all(got[p.n:] == 0x1234)

@@ -97,7 +97,8 @@ namespace ormi::hip {
 
             // Adds root (a node of the program's space); false, with the
             // program as it was, when it does not belong to it: not of its
-            // forms, no operand in common with what is there, or too large.
+            // forms, no operand in common with what is there, too large, or a
+            // reader of an ARGMAX that is there.
             bool add(const NodePtr& root) {
                 const size_t ni = items.size(), nf = frontier.size();
                 const int nr = reductions;
@@ -220,10 +221,14 @@ namespace ormi::hip {
                 return x.a < 0 ? -1 : push(std::move(x));
             }
             // The item of node n read in form `f` (Keep and Full share a context;
-            // a node may also turn out to be Scalar). -1 past the limits.
+            // a node may also turn out to be Scalar). -1 past the limits and for
+            // an ARGMAX of the program.
             int visit(const NodePtr& n, Form f) {
                 const bool in_kept = f == Kept;
                 if (const int id = index_[in_kept].find(n.get()); id >= 0) {
+                    // An ARGMAX that is a root here is an integer in the kernel.
+                    if (!items[id].leaf && items[id].n->op == OpEnum::ARGMAX) over_ = true;
+                    if (over_) return -1;
                     if (items[id].form != Scalar) touched_ = true;
                     return id;
                 }

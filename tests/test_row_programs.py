@@ -70,6 +70,41 @@ def test_what_is_no_program(ob, cpu):
     assert plan(wide.sum(1), wide.max(1)) is None
 
 
+def of_indices(i, j, x):
+    """Values computed from the indices i and j of rows of x."""
+    return [i / j, i * 0.5, i.astype("float32") + x.max(1), x - i.reshape((x.shape[0], 1)).astype("float32")]
+
+
+def test_an_argmax_is_no_operand(ob, cpu):
+    """What reads an ARGMAX of the program is not part of it: the kernel holds
+    the index as an integer."""
+    x = Tensor(values((40, 72)), "cpu")
+    i, j = x.argmax(1), (-x).argmax(1)
+    assert ob._plan_rows([i._node, j._node]) is not None
+    for q in of_indices(i, j, x):
+        assert ob._plan_rows([i._node, j._node, q._node]) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(40, 72), (70, 301), (3, 2049)])
+def test_values_of_an_argmax_beside_it(hip, shape):
+    """The same results realized with the indices as without: a quotient is not
+    truncated, and one by index 0 is inf or NaN."""
+    x = values(shape, 4)
+    x[0, 0], x[1, 0], x[2, 1] = 9.0, -9.0, 9.0
+    X = Tensor(x, hip)
+    i, j = X.argmax(1), (-X).argmax(1)
+    got = of_indices(i, j, X)
+    realize_all(i, j, *got)
+    a, b = x.argmax(1), (-x).argmax(1)
+    assert np.array_equal(i.numpy(), a) and np.array_equal(j.numpy(), b) and a[0] == 0 and b[1] == 0
+    a32, b32 = a.astype(np.float32), b.astype(np.float32)
+    with np.errstate(divide="ignore", invalid="ignore"):
+        np.testing.assert_allclose(got[0].numpy(), a32 / b32, rtol=4 * EPS32)
+    for t, want in zip(got[1:], (a32 * np.float32(0.5), a32 + x.max(1), x - a32[:, None])):
+        assert np.array_equal(t.numpy(), want)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("shape", SHAPES)

@@ -33,6 +33,10 @@ namespace ormi::hip {
 
     namespace {
         constexpr int kMaxItems = 96;     // nodes of one program
+        // Nodes one root may add, views that only rename a value included. An item
+        // is added after its operands, so this, not kMaxItems, bounds how deep
+        // a walk recurses and how much of a long chain a declined root reads.
+        constexpr int kMaxVisits = 4 * kMaxItems;
         constexpr int kMaxReductions = 12;
         constexpr int kMaxHeld = 8;       // operands that vary along a row
         constexpr size_t kMaxColumns = 4;
@@ -103,6 +107,7 @@ namespace ormi::hip {
                 const size_t ni = items.size(), nf = frontier.size();
                 const int nr = reductions;
                 over_ = touched_ = false;
+                visits_ = 0;
                 int it = -1;
                 bool column = false;
                 if (root->op == OpEnum::SUM && root->parents[0]->view.shape == sp.s && is_column(*root)) {
@@ -149,6 +154,7 @@ namespace ormi::hip {
             };
             Index index_[2];
             bool plan_only_, over_ = false, touched_ = false;
+            int visits_ = 0;  // nodes the current add() has walked
 
             void reindex() {
                 index_[0].clear();
@@ -233,6 +239,10 @@ namespace ormi::hip {
                     return id;
                 }
                 if (over_) return -1;
+                if (++visits_ > kMaxVisits) {
+                    over_ = true;
+                    return -1;
+                }
                 if (n->is_realized()) return leaf(n, in_kept);
                 Form own = form_of(n->view.shape, in_kept);
                 if (f == Keep && own == Full) own = None;

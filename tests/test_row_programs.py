@@ -9,6 +9,8 @@ rows too long for the registers (realized one by one as before).
 
 Sums are checked against float64 within n eps32 sum|v| (any order of fp32
 additions), maxima and argmax exactly (ties, NaN and -inf among the values)."""
+import threading
+
 import numpy as np
 import pytest
 from conftest import fp32_sum_tolerance
@@ -68,6 +70,40 @@ def test_what_is_no_program(ob, cpu):
     assert plan(one.sum(1), one.max(1)) is None
     wide = Tensor(np.ones((2, 40000), np.float32), "cpu")
     assert plan(wide.sum(1), wide.max(1)) is None
+
+
+DEEP = 60000
+
+
+def deep(kind, x):
+    """Roots over a chain of DEEP nodes."""
+    h = x.max(1, keepdims=True) if kind == "views" else x
+    for i in range(DEEP):
+        if kind == "reductions":
+            if i % 4 == 0:  # four nodes a level
+                h = h - h.max(1, keepdims=True) * 0.5
+        elif kind == "views":
+            h = h.reshape(h.shape[:1] if i % 2 == 0 else (h.shape[0], 1))
+        else:
+            h = h + 1.0
+    return {"maps": lambda: [h.sum(1), h.max(1)], "beside": lambda: [x.sum(1), h], "softmax": lambda: [softmax(h)],
+            "reductions": lambda: [h], "views": lambda: [x - h]}[kind]()
+
+
+@pytest.mark.parametrize("kind", ["maps", "beside", "softmax", "reductions", "views"])
+def test_deep_chains_are_declined_on_a_small_stack(ob, cpu, kind):
+    """A chain of any length is looked at as far as a program could reach, not
+    to its end: a thread of 256 KB has the stack for it."""
+    roots = [t._node for t in deep(kind, Tensor(np.ones((8, 64), np.float32), "cpu"))]
+    found = []
+    old = threading.stack_size(256 << 10)
+    try:
+        t = threading.Thread(target=lambda: found.append(ob._plan_rows(roots)))
+        t.start()
+    finally:
+        threading.stack_size(old)
+    t.join()
+    assert found == [None]
 
 
 def of_indices(i, j, x):
@@ -225,6 +261,29 @@ def test_deep_chain_of_rows(hip):
         X = X - X.max(1, keepdims=True) * 0.5
         want = want - want.max(1, keepdims=True) * np.float32(0.5)
     assert np.array_equal(X.numpy(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["maps", "beside", "reductions"])
+def test_deep_chains_realize(hip, kind):
+    """DEEP nodes, one root or two: cut into programs and kernels without
+    recursion per level."""
+    x = values((8, 64), 6)
+    roots = deep(kind, Tensor(x, hip))
+    realize_all(*roots)
+    # 1.0 added DEEP times to sixteenths of magnitude below 8 is exact.
+    if kind == "reductions":
+        want = x.copy()
+        for _ in range(0, DEEP, 4):
+            want = want - want.max(1, keepdims=True) * np.float32(0.5)
+        assert np.array_equal(roots[0].numpy(), want)
+    elif kind == "maps":
+        h = x + np.float32(DEEP)
+        assert np.array_equal(roots[1].numpy(), h.max(1))
+        assert np.all(np.abs(roots[0].numpy() - h.astype(np.float64).sum(1)) <= 64 * EPS32 * h.sum(1))
+    else:
+        assert np.array_equal(roots[1].numpy(), x + np.float32(DEEP))
+        assert np.all(np.abs(roots[0].numpy() - x.astype(np.float64).sum(1)) <= fp32_sum_tolerance(x, 1))
 
 
 @pytest.mark.gpu

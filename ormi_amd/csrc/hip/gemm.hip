@@ -1748,19 +1748,24 @@ static int gemm_packed_locked(const ormi_gemm_desc* d, const Epi& epi, long long
 //     6 x 1544 x 2648 25.8 -> 12.4, 1500^3 47 against 70 us) and 2^33 in fp32
 //     (2047 x 2049 x 1023 150 -> 113.5, 424 x 56 x 248 21.6 -> 6.0, 4095^2 x 1001
 //     280 against 330-409).
-// A forced configuration of the other kernels (their environment variables)
-// keeps them.
+// ORMI_GEMM_DIRECT=0 keeps the other kernels, and so does any of their
+// variables that is set, to its default too. The environment is read last, per
+// call, and only where the sizes say yes: reading the nine variables first cost
+// each product 0.3 us of host time (48 x 197 x 197 x 64 in fp16, a product of
+// the tiles, 11.25 -> 11.5 us a call).
 static bool takes_direct(const ormi_gemm_desc* d, long long batch, bool fast) {
-    for (const char* forced : {"ORMI_GEMM_DMA_CFG", "ORMI_GEMM_F32_DMA_CFG", "ORMI_GEMM_CFG16", "ORMI_GEMM_CFG32", "ORMI_GEMM_DMA",
-                               "ORMI_GEMM_F32_DMA", "ORMI_GEMM_MAX_SPLITS", "ORMI_GEMM_PACK"})
-        if (std::getenv(forced)) return false;
     const long long macs = batch * d->M * d->N * (long long)d->K;
     const long long t128 = batch * ((d->M + 127) / 128) * ((d->N + 127) / 128);
     const bool f32 = d->dtype == ORMI_DTYPE_F32;
-    if (fast && d->K % (f32 ? 32 : 64) == 0)
-        return t128 < (f32 ? compute_units() / 4 : compute_units() / 3) && macs <= (1LL << 31) &&
-               (d->K < 4096 || d->M <= 16 || d->N <= 16);
-    return macs <= (f32 ? 1LL << 33 : 5LL << 29);
+    const bool sizes = fast && d->K % (f32 ? 32 : 64) == 0
+                           ? t128 < (f32 ? compute_units() / 4 : compute_units() / 3) && macs <= (1LL << 31) &&
+                                 (d->K < 4096 || d->M <= 16 || d->N <= 16)
+                           : macs <= (f32 ? 1LL << 33 : 5LL << 29);
+    if (!sizes) return false;
+    for (const char* forced : {"ORMI_GEMM_DMA_CFG", "ORMI_GEMM_F32_DMA_CFG", "ORMI_GEMM_CFG16", "ORMI_GEMM_CFG32", "ORMI_GEMM_DMA",
+                               "ORMI_GEMM_F32_DMA", "ORMI_GEMM_MAX_SPLITS", "ORMI_GEMM_PACK"})
+        if (std::getenv(forced)) return false;
+    return env_cfg("ORMI_GEMM_DIRECT", 1) != 0;
 }
 
 static int gemm_run_locked(const ormi_gemm_desc* d, const Epi& epi, long long batch, bool noalloc, bool packed) {
@@ -1821,8 +1826,7 @@ static int gemm_run_locked(const ormi_gemm_desc* d, const Epi& epi, long long ba
     }
 
     hipError_t e;
-    const int direct_env = env_cfg("ORMI_GEMM_DIRECT", 1);
-    if (direct_env != 0 && !packed && (a_kc || a_mc) && (b_kc || b_nc) && (direct_env == 2 || takes_direct(d, batch, fast))) {
+    if (!packed && (a_kc || a_mc) && (b_kc || b_nc) && takes_direct(d, batch, fast)) {
         const DirectPlan r = gemm_direct_plan(d, batch, a_kc, b_kc);
         if (r.mt > 0) {
             if (r.splits > 1) {

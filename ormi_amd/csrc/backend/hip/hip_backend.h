@@ -67,9 +67,11 @@ namespace ormi::hip {
     bool plan_row_program(const std::vector<NodePtr>& roots, int compute_units, RowPlan* plan);
     // Realizes root (and the reductions it reads) as one; false when it is none.
     bool run_row_program(const NodePtr& root);
+    // Whether a row program over several roots could have root's space.
+    bool starts_row_program(const NodePtr& root);
     // Realizes those of `roots` that share operands in row programs; the others
-    // stay unrealized.
-    void realize_row_groups(const std::vector<NodePtr>& roots);
+    // stay unrealized. False when it realized nothing.
+    bool realize_row_groups(const std::vector<NodePtr>& roots);
 
     // ------------------------------------------------------- scheduler --
     // Realize root on the HIP device: pointwise regions become one fused

@@ -100,7 +100,7 @@ namespace ormi::hip {
             }
 
             // Adds root (a node of the program's space); false, with the
-            // program as it was, when it does not belong to it: not of its
+            // program's items as they were, when it does not belong to it: not of its
             // forms, no operand in common with what is there, too large, or a
             // reader of an ARGMAX that is there.
             bool add(const NodePtr& root) {
@@ -121,6 +121,8 @@ namespace ormi::hip {
                 }
                 const bool ok = it >= 0 && !over_ && (column || !items[it].leaf) && (roots.empty() || touched_) && held() <= kMaxHeld;
                 if (!ok) {
+                    // Boundary marks stay: the caller realizes root next, and it
+                    // reads the values that they make the program store.
                     items.resize(ni);
                     frontier.resize(nf);
                     reductions = nr;
@@ -318,6 +320,9 @@ namespace ormi::hip {
                 return false;
             }
             if (!fusible_interior(*root)) return false;
+            bool open = false;
+            for (const auto& p : root->parents) open = open || !p->is_realized();
+            if (!open) return false;
             SmallSet<Node> seen;
             SmallVec<Node*, 64> stack;
             stack.push_back(root.get());
@@ -469,20 +474,27 @@ namespace ormi::hip {
         return find_space(root, &sp) && realize_rows({root}, sp) && root->is_realized();
     }
 
-    void realize_row_groups(const std::vector<NodePtr>& roots) {
+    bool starts_row_program(const NodePtr& root) {
+        Space sp;
+        const NodePtr& n = root_of(root);
+        return !n->is_realized() && find_space(n, &sp);
+    }
+
+    bool realize_row_groups(const std::vector<NodePtr>& roots) {
+        Space sp;
         std::vector<NodePtr> rest;
         SmallSet<Node> seen;
         for (const auto& r : roots) {
             const NodePtr& n = root_of(r);
             if (!n->is_realized() && n->device.type == DeviceEnum::HIP && seen.insert(n.get())) rest.push_back(n);
         }
+        bool done = false;
         while (rest.size() >= 2) {
             // The first root that has a space takes every other root that
             // shares operands with it; roots left over start again.
-            Space sp;
             size_t seed = 0;
             while (seed < rest.size() && !find_space(rest[seed], &sp)) ++seed;
-            if (seed == rest.size()) return;
+            if (seed == rest.size()) break;
             Builder b(sp);
             std::vector<NodePtr> mine, others(rest.begin(), rest.begin() + seed);
             std::vector<NodePtr> after(rest.begin() + seed + 1, rest.end());
@@ -495,10 +507,12 @@ namespace ormi::hip {
                 *list = std::move(left);
             }
             if (mine.size() >= 2 && b.worthwhile()) {
+                done = true;
                 if (b.frontier.empty()) run(b);
                 else realize_rows(mine, sp);
             }
             rest = std::move(after);  // what came before the seed has no space of its own
         }
+        return done;
     }
 }

@@ -617,7 +617,7 @@ namespace ormi::hip {
         return sc.gemms;
     }
 
-    static std::vector<NodePtr> dependencies(const NodePtr& n);
+    static std::vector<NodePtr> dependencies(const NodePtr& n, bool* rows = nullptr);
 
     // Launch self together with a ready partner from the scope; false (nothing
     // launched) when there is none.
@@ -711,8 +711,13 @@ namespace ormi::hip {
 
     // Nodes that must hold buffers before `n` can run as one step: a row
     // program's leaves, a view's parent, an element-wise region's frontier, the frontier (or the input)
-    // of a reduction, a matmul's operands.
-    static std::vector<NodePtr> dependencies(const NodePtr& n) {
+    // of a reduction, a matmul's operands. *rows is set when they are a row
+    // program's leaves: a node without it cannot become one once they hold
+    // buffers, since every reduction its region reads is among them.
+    static std::vector<NodePtr> dependencies(const NodePtr& n, bool* rows) {
+        auto row_frontier = [&](std::vector<NodePtr>& front) {
+            if (reads_a_reduction(front) && row_program_frontier(n, &front) && rows) *rows = true;
+        };
         if (is_view_op(n->op)) return {n->parents[0]};
         if (fusible_root(*n)) {
             EpilogueMatch m;
@@ -724,14 +729,14 @@ namespace ormi::hip {
             }
             if (const NodePtr r = epilogue_reduction(n)) return dependencies(r);
             std::vector<NodePtr> front = region_frontier(n);
-            if (reads_a_reduction(front)) row_program_frontier(n, &front);
+            row_frontier(front);
             return front;
         }
         if (ops::is_reduction(n->op)) {
             const NodePtr& x = n->parents[0];
             if (fuse_as_prologue(x)) {
                 std::vector<NodePtr> front = region_frontier(x);
-                if (reads_a_reduction(front)) row_program_frontier(n, &front);
+                row_frontier(front);
                 return front;
             }
             return {x};
@@ -739,22 +744,19 @@ namespace ormi::hip {
         return n->parents;
     }
 
-    // One node whose dependencies are realized.
-    static void realize_one(const NodePtr& n) {
+    // One node whose dependencies are realized; rows: they are a row program's
+    // leaves.
+    static void realize_one(const NodePtr& n, bool rows) {
         if (n->device.type != DeviceEnum::HIP) throw std::runtime_error("HIP scheduler: node belongs to another device.");
         if (is_view_op(n->op)) {
             n->data = n->parents[0]->data;
             return;
         }
+        if (rows && run_row_program(n)) return;
         if (fusible_root(*n)) {
-            EpilogueMatch m;
-            if (!match_epilogue(n, m) && !match_cast(n, m) && !epilogue_reduction(n) && reads_a_reduction(region_frontier(n)) && run_row_program(n)) return;
             run_map(n);
             return;
         }
-        if (ops::is_reduction(n->op) && fuse_as_prologue(n->parents[0]) && reads_a_reduction(region_frontier(n->parents[0])) &&
-            run_row_program(n))
-            return;
         if (n->op == OpEnum::MATMUL) {
             // Its operands are realized, and so are the activation's (the same).
             if (const NodePtr a = activation_consumer(n)) {
@@ -774,52 +776,68 @@ namespace ormi::hip {
     void realize(const NodePtr& root) {
         if (!root || root->is_realized()) return;
         ScopeGuard guard(&root, 1);
-        SmallVec<NodePtr, 16> stack;
-        stack.push_back(root);
+        struct Step {
+            NodePtr n;
+            bool rows;
+        };
+        SmallVec<Step, 16> stack;
+        stack.push_back({root, false});
         SmallSet<Node> expanded;
         while (!stack.empty()) {
-            const NodePtr n = stack.back();
+            const NodePtr n = stack.back().n;
             if (n->is_realized()) {
                 stack.pop_back();
                 continue;
             }
             if (expanded.insert(n.get())) {
                 bool pushed = false;
-                for (const auto& d : dependencies(n)) {
+                for (const auto& d : dependencies(n, &stack.back().rows)) {
                     if (d->is_realized()) continue;
-                    stack.push_back(d);
+                    stack.push_back({d, false});
                     pushed = true;
                 }
                 if (pushed) continue;
             }
+            const bool rows = stack.back().rows;
             stack.pop_back();
-            realize_one(n);
+            realize_one(n, rows);
         }
     }
 
     void realize_group(const std::vector<NodePtr>& roots) {
         ScopeGuard guard(roots.data(), roots.size());
-        for (const auto& r : roots)
-            if (r && !r->is_realized() && r->device.type != DeviceEnum::HIP)
-                throw std::runtime_error("HIP scheduler: node belongs to another device.");
-        {
-            std::vector<NodePtr> open;
-            for (const auto& r : roots) {
-                EpilogueMatch m;
-                if (r && !r->is_realized() && !match_epilogue(r, m) && !match_cast(r, m)) open.push_back(r);
-            }
-            if (open.size() >= 2) realize_row_groups(open);
+        // Roots that run as a product's epilogue or cast, matched once.
+        SmallVec<char, 16> gemm;
+        auto is_gemm = [](const NodePtr& r) {
+            EpilogueMatch m;
+            return match_epilogue(r, m) || match_cast(r, m);
+        };
+        size_t open = 0;
+        bool rows = false;
+        for (const auto& r : roots) {
+            const bool live = r && !r->is_realized();
+            if (live && r->device.type != DeviceEnum::HIP) throw std::runtime_error("HIP scheduler: node belongs to another device.");
+            gemm.push_back(live && is_gemm(r));
+            if (!live || gemm.back()) continue;
+            ++open;
+            rows = rows || starts_row_program(r);
+        }
+        bool again = false;
+        if (open >= 2 && rows) {
+            std::vector<NodePtr> list;
+            for (size_t i = 0; i < roots.size(); ++i)
+                if (roots[i] && !roots[i]->is_realized() && !gemm[i]) list.push_back(roots[i]);
+            again = realize_row_groups(list);  // perhaps a product's operand too
         }
         // Element-wise roots with float results that can share one kernel,
         // grouped by shape in first-seen order; everything else realizes alone.
         std::vector<std::pair<std::vector<int>, std::vector<NodePtr>>> groups;
         std::vector<NodePtr> rest;
         std::unordered_set<Node*> seen;
-        for (const auto& r : roots) {
+        for (size_t i = 0; i < roots.size(); ++i) {
+            const NodePtr& r = roots[i];
             if (!r || r->is_realized() || !seen.insert(r.get()).second) continue;
-            if (r->device.type != DeviceEnum::HIP) throw std::runtime_error("HIP scheduler: node belongs to another device.");
-            EpilogueMatch m;
-            if (!fusible_interior(*r) || match_epilogue(r, m) || match_cast(r, m) || epilogue_reduction(r)) {
+            if (!fusible_interior(*r) || (again ? is_gemm(r) : gemm[i] != 0) || epilogue_reduction(r)) {
                 rest.push_back(r);
                 continue;
             }

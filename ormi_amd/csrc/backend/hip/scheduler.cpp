@@ -152,6 +152,26 @@ namespace ormi::hip {
         // after these kernels, so reuse is safe.
     }
 
+    // What a product reads for its operand n: n itself, or x where n is an
+    // unrealized 1 * x with a backward pass's seed and x a dense buffer of n's shape,
+    // the same bits (the gradient of sum(c * w) with respect to c, which c's two
+    // backward products read: a copy of 2048 x 4096 took 13.8 us). n stays
+    // unrealized: one that is asked for gets a buffer of its own, since a
+    // caller may write to a gradient's.
+    static const NodePtr& product_operand(const NodePtr& n) {
+        if (n->is_realized() || n->op != OpEnum::MUL || n->dtype != DType::Float32 || n->device.type != DeviceEnum::HIP) return n;
+        for (int k = 0; k < 2; ++k) {
+            const NodePtr* u = &n->parents[k];
+            const NodePtr& x = n->parents[1 - k];
+            while (!(*u)->is_realized() && is_view_op((*u)->op)) u = &(*u)->parents[0];
+            if (!(*u)->is_realized() || !(*u)->data->one || !x->is_realized()) continue;
+            if (x->data->dtype == DType::Float32 && x->device.type == DeviceEnum::HIP && x->view.shape == n->view.shape &&
+                x->view.strides == calc_contiguous_strides(n->view.shape) && (long long)x->data->numel() == shape_numel(n->view.shape))
+                return x;
+        }
+        return n;
+    }
+
     // Operand of a GEMM in the form ormi_hip_gemm takes: dtype f32/bf16/f16,
     // realized. Other dtypes (and mixed pairs) are converted to f32 by a fused
     // cast kernel.
@@ -169,7 +189,7 @@ namespace ormi::hip {
     // (converting other dtypes); `hold` keeps the nodes whose buffers the
     // descriptor points at.
     static ormi_gemm_desc gemm_desc(const NodePtr& root, float* out, std::vector<NodePtr>& hold) {
-        NodePtr A = root->parents[0], B = root->parents[1];
+        NodePtr A = product_operand(root->parents[0]), B = product_operand(root->parents[1]);
         realize(A);
         realize(B);
         DType dt = A->data->dtype;
@@ -253,8 +273,8 @@ namespace ormi::hip {
     // MATMUL on the HIP device (replaces cuda::matmul, csrc/backend/cuda/kernels/blas/
     // matmul.cu:19-122).
     static void prepare_matmul(const NodePtr& root, PreparedGemm& pg) {
-        realize(root->parents[0]);
-        realize(root->parents[1]);
+        realize(product_operand(root->parents[0]));
+        realize(product_operand(root->parents[1]));
         pg.n = root;
         pg.out = empty(root->view.shape, DeviceEnum::HIP, DType::Float32);
         pg.empty = pg.out->numel() == 0;
@@ -659,26 +679,6 @@ namespace ormi::hip {
         return false;
     }
 
-    // A product with a backward pass's seed, 1 * x with x a dense buffer of the
-    // product's shape, is x bit for bit: it aliases x's buffer instead of copying it
-    // (the gradient of sum(c * w) with respect to c, before c's own backward
-    // products: 13.8 us for 2048 x 4096).
-    static bool alias_times_one(const NodePtr& root) {
-        if (root->op != OpEnum::MUL || root->dtype != DType::Float32) return false;
-        for (int k = 0; k < 2; ++k) {
-            const NodePtr &u = root->parents[k], &x = root->parents[1 - k];
-            if (!u->is_realized() || !u->data->one || !x->is_realized()) continue;
-            if (x->data->dtype != DType::Float32 || x->device.type != DeviceEnum::HIP || x->view.shape != root->view.shape ||
-                x->view.strides != calc_contiguous_strides(root->view.shape) ||
-                (long long)x->data->numel() != shape_numel(root->view.shape))
-                continue;
-            root->data = x->data;
-            root->view.strides = x->view.strides;
-            return true;
-        }
-        return false;
-    }
-
     // An element-wise region: a matched GEMM epilogue, a reduction's store
     // epilogue, else one fused kernel.
     static void run_map(const NodePtr& root) {
@@ -692,7 +692,6 @@ namespace ormi::hip {
             return;
         }
         for (const auto& f : region_frontier(root)) realize(f);
-        if (alias_times_one(root)) return;
         const Expr e = build_expr(root, root->view.shape);
         auto out = empty(root->view.shape, DeviceEnum::HIP, root->dtype);
         root->data = out;
@@ -722,7 +721,7 @@ namespace ormi::hip {
         if (fusible_root(*n)) {
             EpilogueMatch m;
             if (match_epilogue(n, m) || match_cast(n, m)) {
-                std::vector<NodePtr> deps{m.g->parents[0], m.g->parents[1]};
+                std::vector<NodePtr> deps{product_operand(m.g->parents[0]), product_operand(m.g->parents[1])};
                 if (m.d) deps.push_back(m.d);
                 if (m.s) deps.push_back(m.s);
                 return deps;
@@ -741,6 +740,7 @@ namespace ormi::hip {
             }
             return {x};
         }
+        if (n->op == OpEnum::MATMUL) return {product_operand(n->parents[0]), product_operand(n->parents[1])};
         return n->parents;
     }
 

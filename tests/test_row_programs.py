@@ -9,6 +9,7 @@ rows too long for the registers (realized one by one as before).
 
 Sums are checked against float64 within n eps32 sum|v| (any order of fp32
 additions), maxima and argmax exactly (ties, NaN and -inf among the values)."""
+import ctypes
 import threading
 
 import numpy as np
@@ -284,6 +285,37 @@ def test_deep_chains_realize(hip, kind):
     else:
         assert np.array_equal(roots[1].numpy(), x + np.float32(DEEP))
         assert np.all(np.abs(roots[0].numpy() - x.astype(np.float64).sum(1)) <= fp32_sum_tolerance(x, 1))
+
+
+@pytest.mark.gpu
+def test_a_gradient_owns_its_buffer(hip, cabi):
+    """1 * w as a gradient is a copy of w, asked for first, last or after the
+    products that read w in its place: filling it leaves w as it was."""
+    rng = np.random.default_rng(8)
+    a, b, w = (rng.standard_normal(s).astype(np.float32) for s in ((40, 24), (24, 56), (40, 56)))
+    W, nine = Tensor(w, hip), np.array([9], np.float32)
+
+    def fill(t):
+        assert np.array_equal(t.numpy(), w) and t._node.data.ptr != W._node.data.ptr
+        assert cabi.ormi_hip_fill(ctypes.c_void_p(t._node.data.ptr), nine.ctypes.data, 4, w.size) == 0
+        assert np.array_equal(t.numpy(), np.full_like(w, 9)) and np.array_equal(W.numpy(), w)
+
+    X = Tensor(w * 2, hip, requires_grad=True)
+    (X * W).sum().backward()
+    fill(X.grad)
+    for first in (True, False):
+        A, B = Tensor(a, hip, requires_grad=True), Tensor(b, hip, requires_grad=True)
+        C = A @ B
+        total = (C * W).sum()
+        total.backward()
+        if first:
+            realize_all(C.grad, A.grad, B.grad)
+        else:
+            realize_all(A.grad, B.grad)
+        assert np.all(np.abs(A.grad.numpy() - w.astype(np.float64) @ b.T) <= 60 * EPS32 * (np.abs(w) @ np.abs(b).T))
+        assert np.all(np.abs(B.grad.numpy() - a.T.astype(np.float64) @ w) <= 60 * EPS32 * (np.abs(a).T @ np.abs(w)))
+        fill(C.grad)
+        total.zero_grad_graph()
 
 
 @pytest.mark.gpu

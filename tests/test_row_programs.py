@@ -163,6 +163,22 @@ def test_stats(ob, hip, shape, dtype):
 
 
 @pytest.mark.gpu
+def test_waves_of_a_row_add_pairwise(ob, hip):
+    """Sixteen waves share a row, one group of four per lane: 2 + 6 + 4 levels of
+    additions, each off by at most half an ulp of the row's sum. One wave's sum
+    after the other would lose all fifteen ones against 2^24."""
+    x = np.zeros((8, 4096), np.float32)
+    x[:, 256::256] = 1.0
+    x[:, 0] = 2.0 ** 24
+    X = Tensor(x, hip)
+    s, top = X.sum(1), X.max(1)
+    assert "lanes=1024 groups=1" in ob._plan_rows([s._node, top._node])["plan"]
+    realize_all(s, top)
+    exact = x.astype(np.float64).sum(1)
+    assert np.all(np.abs(s.numpy() - exact) <= 12 * EPS32 / 2 * exact) and np.all(top.numpy() == 2.0 ** 24)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("shape", SHAPES)
 def test_special_values(hip, shape):
     """Rows of -inf only, with inf, and with NaN: the first NaN is the maximum."""

@@ -141,12 +141,14 @@ int ormi_hip_rtc_cache_size(uint64_t* entries);
  * A[m][k] lives at a + m*a_stride_m + k*a_stride_k (elements); normally one of
  * the two strides is 1 (stride_k == 1: "N", stride_m == 1: "T", the reference's
  * trans rule matmul.cu:47-52). Same for B with (stride_k, stride_n). Other
- * strides are accepted. Unit-stride operands of any alignment and extent run
- * on matrix-core kernels as they are up to 2.7e9 multiply-adds (fp32 2^33);
- * larger products whose operands are not in whole 16-byte chunks, and large
- * ones with no unit stride, are first copied into a zero-padded, k-contiguous
- * device buffer the library keeps and grows on demand; the rest run a generic
- * kernel.
+ * strides are accepted. Unit-stride operands run on matrix-core kernels as they
+ * are, of any alignment too where that is the faster way (up to 2^31
+ * multiply-adds, fp32 2^33; not a short K, and not an operand contiguous along m
+ * or n with fewer than 2 to 4 elements there). Other products of 2^24
+ * multiply-adds or more whose operands are not in whole 16-byte chunks or have no
+ * unit stride are first copied into a zero-padded, k-contiguous device buffer
+ * the library keeps and grows on demand (not by ormi_hip_gemm_ex_noalloc); the
+ * rest run a generic kernel.
  * C is written contiguous: C[b][m][n] at c + b*M*N + m*N + n, fp32.
  * dtype: ORMI_DTYPE_F32 (fp32 MFMA), ORMI_DTYPE_BF16 or ORMI_DTYPE_F16
  * (MFMA with fp32 accumulation). Batch index b decomposes row-major over

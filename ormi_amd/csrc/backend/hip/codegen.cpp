@@ -2068,12 +2068,8 @@ namespace ormi::hip {
         KernelLaunch& s2 = plan->second;
         Gen g2(no_expr());
         g2.args.ptr(true, "float", "part", nullptr);
-        int j2 = 0;
         for (size_t r = 0; r < nout; ++r)
-            if (prog.out_kinds[r] == RowOut::Column) {
-                g2.args.ptr(false, "float", "out", prog.outs[r], (int)r);
-                ++j2;
-            }
+            if (prog.out_kinds[r] == RowOut::Column) g2.args.ptr(false, "float", "out", prog.outs[r], (int)r);
         g2.args.i64("NR", R);
         g2.args.i64("NP", grid);
         s2.grid[0] = (uint32_t)((R + 63) / 64);

@@ -125,11 +125,17 @@ namespace ormi::hip {
         // kernels whose such leaves bring in at least this many bytes.
         long long nt_min_bytes = 64LL << 20;
         // Row programs. Registers per lane for held operands and column sums, at
-        // most rows_groups groups of each. Work-groups per compute unit without
-        // column sums (no limit in practice) and with them: every work-group then
-        // leaves one partial row, and 3 measured best on 16384 x 8192 (row
-        // kernel + finish: 2: 109 + 6.0, 3: 97 + 8.7, 4: 101 + 11.1, 5: 109 + 13.6
-        // us with the first finish kernel; 512 threads, 2: 111 + 5.9).
+        // most rows_groups groups of each; not scaled by the work-group, so with 1024
+        // threads (128 registers a lane) wide rows of many operands spill: a
+        // normalization forward and backward over 16384 and 20480 columns, 92 and
+        // 192 bytes a lane (12288: none), and still 2.0 and 1.7 times as fast as its
+        // kernels one by one (4096 rows, 276 and 450 us a call against 553 and 777).
+        // Work-groups per compute unit without column sums (no limit in practice) and
+        // with them: every work-group then leaves one partial row. 3 was measured on
+        // 16384 x 8192 alone, where a lane has 124 registers (row kernel + finish:
+        // 2: 109 + 6.0, 3: 97 + 8.7, 4: 101 + 11.1, 5: 109 + 13.6 us with the first
+        // finish kernel; 512 threads, 2: 111 + 5.9); narrow rows use fewer registers
+        // and might do better with more.
         int rows_regs = 128;
         int rows_groups = 8;
         int rows_wg_per_cu = 4096;

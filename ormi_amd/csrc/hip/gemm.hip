@@ -3,6 +3,8 @@
 // cublasSgemmBatched call (csrc/backend/cuda/kernels/blas/matmul.cu:98-105).
 //
 // Kernels, in the order the dispatch (gemm_run_locked) prefers them
+//   * Register-fragment kernels (gemm_direct.hip): few rows or columns, small
+//     matrices, operands not in whole 16-byte chunks (takes_direct).
 //   * 16-bit direct-load kernels (this file): HBM -> LDS with
 //     global_load_lds_dwordx4 into XOR-swizzled multi-stage rings, 4 waves of
 //     128x128 (256x256 tiles) or 64x64 (128x128 tiles), 32x32x16 MFMAs. A
@@ -23,8 +25,8 @@
 //     unpackable layouts).
 // Shared by all
 //   * An element-wise epilogue (ormi_hip_gemm_ex) is applied in the store of
-//     the fp32 direct-load kernels (gemm_f32dma.hip, gemm_epi.hip), otherwise
-//     in the pass that finishes a K split.
+//     the register-fragment and the fp32 direct-load kernels (gemm_f32dma.hip,
+//     gemm_epi.hip), otherwise in the pass that finishes a K split.
 //   * The tile index is remapped so the 8 XCDs (round-robin block dispatch)
 //     each own a compact group of tiles, sharing operand panels in their L2.
 //   * When the output has too few tiles to occupy the 256 CUs, K is split
@@ -1733,39 +1735,85 @@ static int gemm_packed_locked(const ormi_gemm_desc* d, const Epi& epi, long long
     return gemm_run_locked(&dp, epi, batch, false, true);
 }
 
-// Whether gemm_direct.hip's kernels take a product (both operands unit-stride
-// in one index). Measured against the kernels that would run otherwise, on
-// about 80 shapes from 1 x 1 x 5000 to 4095^3, operands rotating through memory:
-//   * operands in whole 16-byte chunks with K in whole k-tiles, where the
-//     direct-load tiles run: while those tiles number under a third (fp32: a
-//     quarter) of the compute units, up to 2^31 multiply-adds (1024^3 bf16
-//     17.6 -> 12.0 us, 512^3 8.8 -> 5.4, 12 x 8192 x 2048 15.1 -> 12.3; past the
-//     line 2048^3 26 against 59, 200 x 4096^2 22 against 44, fp32 1024^3 26.6
-//     against 25.7), except where K is long enough to feed the tiles' splits
-//     (40 x 4096^2 16.1 against 18.2, 64 x 1024 x 8192 13.0 against 14.1);
-//   * otherwise packing, the register-staged kernels or the generic one would
-//     run: up to 2.7e9 multiply-adds in 16 bits (1001 x 1003 x 1005 34.4 -> 20.2,
-//     6 x 1544 x 2648 25.8 -> 12.4, 1500^3 47 against 70 us) and 2^33 in fp32
-//     (2047 x 2049 x 1023 150 -> 113.5, 424 x 56 x 248 21.6 -> 6.0, 4095^2 x 1001
-//     280 against 330-409).
+// Whether gemm_direct.hip's kernels take a product, with plan r for it. Each
+// line below lies where they and the kernels that would run otherwise cross:
+// both were timed on 15500 random products (fp32, bf16 and fp16; every layout;
+// one matrix and batches; extents 1 to 8192), operands rotating through memory.
+//   * K in whole tiles, 16-byte chunks (the direct-load tiles run otherwise).
+//     Fewer than a third (fp32: a quarter) of the compute units' worth of 128 x 128
+//     tiles, up to 2^31 multiply-adds (2048^3 26 against 59 us), and
+//       - a K deep enough for a few steps per wave: 8 x 16 x 32-deep fp32 tiles lose
+//         5-15% at K = 32, 16-bit ones at 64;
+//       - at most one work-group per compute unit: a second round of them waits
+//         for the first (fp32 1016 x 704 x 1088 28 against 35). In 16 bits up to two,
+//         where K is so long that the tiles would split it, or A is read
+//         along m, which the tiles are slower at (1016 x 992 x 576 16.1 -> 8.7);
+//       - not a long K, on which the tiles' split K is the better one (bf16 816 x
+//         1344 x 1728 19.4 against 27.0, fp32 120 x 1192 x 3936 26.9 against 38.8),
+//         unless there are few rows or columns, the chip is filled by small
+//         tiles (fp32 336 x 232 x 896 16.1 -> 10.8) or nearly by large ones.
+//     Up to 16 rows: every K in fp32 (1.3-3.4 times as fast); 16 bits leaves out
+//     two splits with three steps a wave or more, or with few tiles (7 x 4032 x 3712
+//     13.6 against 16.7), and four with few tiles of deep weights.
+//   * 16-byte chunks, but K in part of a tile (register-staged kernels): all but
+//     several rounds of work-groups with a k-contiguous B or a short K (922 x 708 x 24
+//     in 42 batches, 36.5 against 53.4).
+//   * Otherwise packing or the generic kernel would run. Below 2^24 multiply-adds
+//     the generic one, which has no partial k-step to load element by element:
+//     the better one up to K of about 128 (16 bits 160; bf16 192 x 25 x 26 3.8 against
+//     6.6). Above, up to 2^33 in fp32 and 2^31 in 16 bits (4095^2 x 1001 fp32
+//     280 against 330-409, 1001 x 1003 x 1005 bf16 34.4 -> 20.2); a k-contiguous B is
+//     read in strides by its rows, so that packing it pays from 2^31 and 2^30
+//     (bf16 420 x 2011 x 1943 35 against 64).
+// On 4000 more, these lines are 1.28-2.3 times as fast as the other kernels alone in
+// the geometric mean (few rows of 16 bits with K from 1792: 1.05), 3% of them
+// slower by more than 3% and one in 500 by more than 12%. Lines that had been drawn
+// on 80 shapes had 15-30% slower, down to 0.44 times the speed.
 // ORMI_GEMM_DIRECT=0 keeps the other kernels, and so does any of their
-// variables that is set, to its default too. The environment is read last, per
-// call, and only where the sizes say yes: reading the nine variables first cost
-// each product 0.3 us of host time (48 x 197 x 197 x 64 in fp16, a product of
-// the tiles, 11.25 -> 11.5 us a call).
-static bool takes_direct(const ormi_gemm_desc* d, long long batch, bool fast) {
-    const long long macs = batch * d->M * d->N * (long long)d->K;
-    const long long t128 = batch * ((d->M + 127) / 128) * ((d->N + 127) / 128);
+// variables that is set, to its default too; 2 takes every product with a plan.
+// Those variables are read last, per call, and only where the sizes say yes:
+// reading all first cost each product 0.3 us of host time (48 x 197 x 197 x 64 in
+// fp16, a product of the tiles, 5.29 -> 5.00 us to enqueue).
+static bool direct_sizes(const ormi_gemm_desc* d, long long batch, bool fast, const DirectPlan& r, bool a_kc, bool b_kc) {
     const bool f32 = d->dtype == ORMI_DTYPE_F32;
-    const bool sizes = fast && d->K % (f32 ? 32 : 64) == 0
-                           ? t128 < (f32 ? compute_units() / 4 : compute_units() / 3) && macs <= (1LL << 31) &&
-                                 (d->K < 4096 || d->M <= 16 || d->N <= 16)
-                           : macs <= (f32 ? 1LL << 33 : 5LL << 29);
-    if (!sizes) return false;
+    const long long M = d->M, N = d->N, K = d->K, cus = compute_units(), macs = batch * M * N * K;
+    const long long tiles = batch * ((M + 16 * r.mt - 1) / (16 * r.mt)) * ((N + 16 * r.nt - 1) / (16 * r.nt));
+    const long long groups = tiles * r.splits;
+    if (fast && K % (f32 ? 32 : 64) == 0) {
+        const long long t128 = batch * ((M + 127) / 128) * ((N + 127) / 128);
+        if (t128 >= (f32 ? cus / 4 : cus / 3) || macs > (1LL << 31) || (K >= 4096 && M > 16 && N > 16)) return false;
+        if (f32) {
+            if (K < 64) return false;
+            if (M <= 16) return true;
+            if (N <= 16) return K <= 768 || K % 64 == 0;
+            if (groups > cus) return false;
+            if (K <= 768 || (M <= 32 && (K % 64 == 0 || macs > (1LL << 26)))) return true;
+            const double steps = (double)K / (16.0 * r.waves * r.splits);  // per wave
+            if (r.mt * r.nt <= 4) return (K % 64 == 0 || K < 1152) && steps <= 6;
+            return r.splits == 1 && groups >= 11 * cus / 16 && steps <= 12;
+        }
+        if (K < 128) return false;
+        if (M <= 16)
+            return groups <= cus && !(r.splits == 2 && K < 4096 && (K >= 3072 || tiles < cus / 8)) &&
+                   !(r.nt == 4 && r.splits == 4 && tiles < 11 * cus / 64);
+        if (K > 1792 || (N <= 16 && (K < 256 || K > 1024))) return false;
+        return groups <= cus || (groups <= 2 * cus && K <= 1024 && K >= (a_kc ? 512 : 256));
+    }
+    if (macs > (f32 ? 1LL << 33 : 1LL << 31)) return false;
+    if (fast) return groups <= cus || (!b_kc && K >= 128);
+    if (macs < (1LL << 24)) return K >= (f32 ? 128 : 160);
+    if (macs < (1LL << 25) && K < 64) return false;
+    return !b_kc || M * N * K < (1LL << 24) || macs <= (f32 ? 1LL << 31 : 1LL << 30);
+}
+static bool takes_direct(const ormi_gemm_desc* d, long long batch, bool fast, const DirectPlan& r, bool a_kc, bool b_kc) {
+    if (r.mt == 0) return false;
+    const int mode = env_cfg("ORMI_GEMM_DIRECT", 1);
+    if (mode == 2) return true;
+    if (mode == 0 || !direct_sizes(d, batch, fast, r, a_kc, b_kc)) return false;
     for (const char* forced : {"ORMI_GEMM_DMA_CFG", "ORMI_GEMM_F32_DMA_CFG", "ORMI_GEMM_CFG16", "ORMI_GEMM_CFG32", "ORMI_GEMM_DMA",
                                "ORMI_GEMM_F32_DMA", "ORMI_GEMM_MAX_SPLITS", "ORMI_GEMM_PACK"})
         if (std::getenv(forced)) return false;
-    return env_cfg("ORMI_GEMM_DIRECT", 1) != 0;
+    return true;
 }
 
 static int gemm_run_locked(const ormi_gemm_desc* d, const Epi& epi, long long batch, bool noalloc, bool packed) {
@@ -1826,9 +1874,9 @@ static int gemm_run_locked(const ormi_gemm_desc* d, const Epi& epi, long long ba
     }
 
     hipError_t e;
-    if (!packed && (a_kc || a_mc) && (b_kc || b_nc) && takes_direct(d, batch, fast)) {
+    if (!packed && (a_kc || a_mc) && (b_kc || b_nc)) {
         const DirectPlan r = gemm_direct_plan(d, batch, a_kc, b_kc);
-        if (r.mt > 0) {
+        if (takes_direct(d, batch, fast, r, a_kc, b_kc)) {
             if (r.splits > 1) {
                 void* ws = nullptr;
                 rc = workspace((size_t)batch * d->M * d->N * r.splits * sizeof(float), &ws);

@@ -7,8 +7,12 @@
 // from memory into registers, from any element address, so there is no tile to
 // fill, no alignment to meet and no barrier in the main loop: a wave computes
 // 16 MT x 16 NT elements over a share of K, the W waves of a work-group split K
-// among them, and their partial tiles are added through LDS in a fixed tree.
-// No workspace and no second kernel: the first wave applies the epilogue.
+// among them, and their partial tiles meet in LDS, where each wave adds some of
+// the tile's rows in wave order, applies the epilogue and stores them. So most
+// products need no workspace and no second kernel. Where the tiles leave a
+// quarter of the chip idle and K is long, up to 8 work-groups share a tile's K:
+// their tiles go to a workspace, and the finish pass (gemm.hip) adds them in
+// split order and applies the epilogue.
 //
 // Fragments. A 16 x 16 MFMA takes, per lane, KV consecutive k of one row of A
 // and one column of B (KV = 8 values of 16 bits, 4 floats for four K = 4
@@ -353,7 +357,8 @@ void launch_cfg(int mt, int nt, const GemmParams& p, dim3 grid, int waves, bool 
 }  // namespace
 
 // Tile (in 16-element fragments) and waves per work-group for a product, or
-// mt = 0 when an mn-contiguous operand has fewer elements than a fragment load.
+// mt = 0 when an mn-contiguous operand has fewer rows (columns) than a fragment
+// load takes, up to 4: the other kernels run it.
 DirectPlan gemm_direct_plan(const ormi_gemm_desc* d, long long batch, bool a_kc, bool b_kc) {
     DirectPlan r;
     const long long cus = compute_units();

@@ -92,8 +92,11 @@ class Product:
         assert np.all(np.abs(got - want) <= self.bound * (1 + extra) + extra * EPS32 * (1 + np.abs(want)))
 
 
-@pytest.fixture
-def product(cabi):
+@pytest.fixture(params=["by size", "always"])
+def product(cabi, request, monkeypatch):
+    """By size: the kernels that the dispatch takes. Always: those of
+    gemm_direct.hip wherever they can run (ORMI_GEMM_DIRECT, read per call)."""
+    monkeypatch.setenv("ORMI_GEMM_DIRECT", "1" if request.param == "by size" else "2")
     made = []
 
     def make(*a, **k):

@@ -534,8 +534,13 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(GemmParams p) {
         As[ty][tx] = (ar < p.M && ak < p.K) ? gemm_elem<DT>(p.a, a_off + (long long)ar * p.a_sm + (long long)ak * p.a_sk) : 0.0f;
         Bs[ty][tx] = (bk < p.K && bc < p.N) ? gemm_elem<DT>(p.b, b_off + (long long)bk * p.b_sk + (long long)bc * p.b_sn) : 0.0f;
         __syncthreads();
+        // Four chains of four, added pairwise: one chain through K had 1.3 to 2.2
+        // times the register-fragment kernels' error at K below 128, where
+        // products come here from them (direct_sizes).
+        float t[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int kk = 0; kk < 16; ++kk) acc = __builtin_fmaf(As[ty][kk], Bs[kk][tx], acc);
+        for (int kk = 0; kk < 16; ++kk) t[kk % 4] = __builtin_fmaf(As[ty][kk], Bs[kk][tx], t[kk % 4]);
+        acc += (t[0] + t[1]) + (t[2] + t[3]);
         __syncthreads();
     }
     if (row < p.M && col < p.N) {

@@ -253,3 +253,24 @@ def test_cast_of_a_batch_is_laid_out_like_c(hip, product, cabi, dtype, cast_dtyp
     p.check(c, np.maximum(p.exact, 0))
     got = p.dev.get(out, (p.n + 8) * 2).view(np.uint16)
     assert np.array_equal(got[:p.n], storage(c.reshape(-1), cast_dtype)[0].view(np.uint16)) and np.all(got[p.n:] == 0x1234)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [F32, BF16, F16])
+def test_generic_kernel_adds_in_short_chains(hip, cabi, monkeypatch, dtype):
+    """K = 96 in six steps of four chains of four: 3 + 2 + 6 additions after the
+    largest term, 2^24, each off by at most half an ulp, 1. One chain through K
+    would lose all 95 ones."""
+    monkeypatch.setenv("ORMI_GEMM_DIRECT", "0")
+    M, N, K = 3, 5, 96
+    p = Product(cabi, dtype, "nn", M, N, K)
+    try:
+        a, b = np.ones((M, K), np.float32), np.ones((K, N), np.float32)
+        a[:, 0], b[0] = 2.0 ** 12, 2.0 ** 12
+        for dst, x in ((p.d.a, a), (p.d.b, b)):
+            bits = np.ascontiguousarray(storage(x, dtype)[0])
+            assert cabi.ormi_hip_memcpy_h2d(ctypes.c_void_p(dst), bits.ctypes.data, bits.nbytes) == 0
+        p.run()
+        assert np.all(np.abs(p.get().astype(np.float64) - (2.0 ** 24 + K - 1)) <= 11)
+    finally:
+        p.dev.free()

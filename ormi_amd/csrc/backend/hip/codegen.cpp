@@ -378,8 +378,9 @@ namespace ormi::hip {
             // bfloat16: 6001 x 2047 26.7 us with one element per lane, 15.4 in
             // groups, the time of 6001 x 2048 (both bound by the arithmetic). ragged_ok: the
             // caller handles an extent that is not a multiple of four (tail).
+            // any_address: groups pay from addresses that are not multiples of them.
             static constexpr long long kRaggedMin = 256 * 4 * 64;
-            void choose_vec(int d, bool ragged_ok) {
+            void choose_vec(int d, bool ragged_ok, bool any_address = true) {
                 vec = 1;
                 vec_dim = d;
                 tail = false;
@@ -401,7 +402,7 @@ namespace ormi::hip {
                 // groups 5.4).
                 long long numel = 1;
                 for (auto& x : c.dims) numel *= x.size;
-                if (any && numel < kRaggedMin) {
+                if (any && (numel < kRaggedMin || !any_address)) {
                     tail = false;
                     unaligned.assign(e.leaves.size(), false);
                     return;
@@ -1193,9 +1194,17 @@ namespace ormi::hip {
         const bool column = !id.empty();
         // A ragged vector dim must be the only dim of its group: positions
         // within the group are then group starts plus the lane's slot.
-        // Fewer than 16 ragged columns keep one lane per column.
-        if (column) g.choose_vec(id.back(), id.size() == 1 && I >= 16);
-        else g.choose_vec(rd.empty() ? -1 : rd.back(), rd.size() == 1);
+        // Where rows start at any element, groups leave a quarter of the lanes
+        // to read the row, so they pay only where the lanes stay busy (1320
+        // ragged shapes both ways): rows from 160 elements, but of more than
+        // 4096 rows not those that fill a wave's second pass or its fourth by less
+        // than half (58543 x 5 12.5 us against 18.3, 13948 x 791 7.7 against 11.1;
+        // with groups 300 x 27000 ran up to 1.3, rows of 160 to 256 up to 2.1 times
+        // as fast); columns from 64 to 2048 of 2^21 elements or more (47 x 3251 6.6
+        // against 11.4; with groups up to 2.0 times).
+        const bool row_groups = R >= 160 && (O <= 4096 || !((R > 256 && R <= 384) || (R > 768 && R <= 1024)));
+        if (column) g.choose_vec(id.back(), id.size() == 1, I >= 64 && I <= 2048 && O * R * I >= (1LL << 21));
+        else g.choose_vec(rd.empty() ? -1 : rd.back(), rd.size() == 1, row_groups);
 
         ReducePlan plan;
         KernelLaunch& k = plan.first;

@@ -21,13 +21,25 @@ SHAPES = [(1, 5), (7, 7), (2, 1021), (129, 66), (2, 3, 5), (16384, 5), (9363, 7)
           (17, 4099), (1009, 66), (4099, 17), (4, 9, 2050), (16, 1025, 5)]
 
 
-@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("shape", SHAPES + [(58543, 5), (5000, 301), (4000, 301), (5000, 401), (13948, 791), (4000, 791), (420, 163)])
 def test_ragged_group_kernels_plan_vectors(ob, cpu, shape):
-    """Ragged rows take groups of four from 256 x 4 x 64 elements up (no GPU)."""
+    """Ragged rows take groups of four from 256 x 4 x 64 elements up; a reduction's
+    from 160 elements a row, and of many rows only those that keep its waves
+    busy (no GPU)."""
     x, b = (Tensor(np.zeros(s, np.float32), "cpu") for s in (shape, shape[-1:]))
-    vec = "vec=4" if np.prod(shape) >= 65536 else "vec=1"
-    assert vec in ob._plan_kernel(((x + b) * 2.0)._node)["plan"]
-    assert vec in ob._plan_kernel(ob.sum(x._node, [len(shape) - 1], False))["plan"]
+    rows, cols = int(np.prod(shape[:-1])), shape[-1]
+    large = rows * cols >= 65536
+    assert ("vec=4" if large else "vec=1") in ob._plan_kernel(((x + b) * 2.0)._node)["plan"]
+    groups = large and cols >= 160 and (rows <= 4096 or not (256 < cols <= 384 or 768 < cols <= 1024))
+    assert ("vec=4" if groups else "vec=1") in ob._plan_kernel(ob.sum(x._node, [len(shape) - 1], False))["plan"]
+
+
+@pytest.mark.parametrize("shape,groups", [((16384, 129), True), ((33000, 65), True), ((33500, 63), False), ((16384, 127), False), ((47, 3251), False),
+                                          ((1030, 2047), True), ((1100, 2049), False)])
+def test_ragged_columns_plan_vectors(ob, cpu, shape, groups):
+    """64 to 2048 ragged columns of 2^21 elements or more (no GPU)."""
+    x = Tensor(np.zeros(shape, np.float32), "cpu")
+    assert ("vec=4" if groups else "vec=1") in ob._plan_kernel(ob.sum(x._node, [0], False))["plan"]
 
 
 @pytest.mark.gpu
@@ -51,7 +63,7 @@ def test_ragged_maps_match_oracle(cpu, hip, shape, dtype):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
-@pytest.mark.parametrize("shape", SHAPES + [(5000, 5), (4099, 301), (70000, 17), (301, 4099), (66, 20001)])
+@pytest.mark.parametrize("shape", SHAPES + [(5000, 5), (4099, 301), (70000, 17), (301, 4099), (66, 20001), (4200, 501), (2, 16384, 65)])
 def test_ragged_reductions(hip, shape, dtype):
     rng = np.random.default_rng(int(np.prod(shape)) + 1)
     x = np.round(rng.standard_normal(shape) * 16).astype(np.float32) / 16  # exact in bfloat16, with ties

@@ -179,6 +179,23 @@ def test_waves_of_a_row_add_pairwise(ob, hip):
 
 
 @pytest.mark.gpu
+def test_column_sums_of_work_groups_add_pairwise(ob, hip):
+    """One row per work-group, so 256 parts per column: 4 + 4 levels of additions,
+    each off by at most half an ulp of the column's sum. One part after the other
+    would lose the fifteen ones of the first wave's parts against 2^24, one wave
+    after the other the fifteen of the other waves."""
+    x = np.zeros((256, 4096), np.float32)
+    x[1:16], x[16::16] = 1.0, 1.0
+    x[0] = 2.0 ** 24
+    X = Tensor(x, hip)
+    s, top = X.sum(0), X.max(1)
+    assert "O=256 R=4096 vec=4 lanes=256" in ob._plan_rows([s._node, top._node])["plan"]
+    realize_all(s, top)
+    exact = x.astype(np.float64).sum(0)
+    assert np.all(np.abs(s.numpy() - exact) <= 8 * EPS32 / 2 * exact) and np.all(top.numpy() == x.max(1))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("shape", SHAPES)
 def test_special_values(hip, shape):
     """Rows of -inf only, with inf, and with NaN: the first NaN is the maximum."""
